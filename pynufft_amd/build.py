@@ -12,7 +12,9 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB = os.path.join(HERE, 'libpynufft_hip.so')
-SOURCES = ['api.hip', 'fft.hip', 'interp.hip', 'vec.hip', 'solvers.hip']
+# source, object, extra flags; the FFT lengths' kernels in parts (PNH_CT_PARTS)
+SOURCES = [(s + '.hip', s + '.o', []) for s in ('interp', 'api', 'fft', 'vec', 'solvers')] + \
+    [('fft_ct.hip', 'fft_ct%d.o' % k, ['-DPNH_CT_PART=%d' % k]) for k in range(7)]
 ARCH = os.environ.get('PYNUFFT_HIP_ARCH', 'gfx950')
 
 
@@ -31,16 +33,16 @@ def compile_flags():
             '-Wno-unused-result']
 
 
-def build(verbose=True, jobs=4):
+def build(verbose=True, jobs=8):
     """Compile every source to an object in parallel, then link the .so."""
     objdir = os.path.join(HERE, '_build')
     os.makedirs(objdir, exist_ok=True)
     procs = []
     objs = []
-    for src in SOURCES:
-        obj = os.path.join(objdir, src.replace('.hip', '.o'))
+    for src, obj, extra in SOURCES:
+        obj = os.path.join(objdir, obj)
         objs.append(obj)
-        cmd = [hipcc()] + compile_flags() + ['-c', os.path.join(CSRC, src), '-o', obj]
+        cmd = [hipcc()] + compile_flags() + extra + ['-c', os.path.join(CSRC, src), '-o', obj]
         if verbose:
             print(' '.join(cmd), flush=True)
         procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE,

@@ -43,6 +43,9 @@ struct pnh_plan {
   int J[PNH_MAXD];
   BinArgs bins;
   int slot_nbc;            // coils per partial slot element (min(nb, 4))
+  // [precision][inverse][axis] launch geometry of the FFT passes, made with
+  // the plan (n = 0: a length not supported there, refused when it is used)
+  FftDesc fft[2][2][PNH_MAXD];
 };
 
 namespace {
@@ -83,14 +86,89 @@ size_t partial_bytes(const pnh_plan* p, int fp64) {
          (size_t)p->d.n_slots * p->bins.pad_cells * p->slot_nbc * esz;
 }
 
-// Build the line-FFT descriptor for axis `a`.
+// The launch geometry of the line FFT along axis `a` (radices, lines and
+// threads per workgroup, division multipliers): made once per plan, see
+// pnh_plan::fft.  Returns -2 with the message set when the length is not
+// supported.  compiled: the launch may take the kernel compiled for the length.
+int pass_geometry(const pnh_plan* p, int a, bool inverse, int fp64, FftDesc* f,
+                  bool compiled = true) {
+  memset(f, 0, sizeof(*f));
+  f->n = (int)p->K[a];
+  f->n_in = inverse ? (int)p->K[a] : (int)p->N[a];
+  f->n_out = inverse ? (int)p->N[a] : (int)p->K[a];
+  f->sign = inverse ? 1 : -1;
+  // outer dims: d < a with image extents
+  int64_t n_outer = 1;
+  for (int d = 0; d < a; ++d) n_outer *= p->N[d];
+  f->n_outer = n_outer;
+  f->o_split = (a >= 2) ? p->N[1] : 1;
+  int64_t n_inner = p->nb;
+  for (int d = a + 1; d < p->D; ++d) n_inner *= p->K[d];
+  f->n_inner = n_inner;
+  if (pnh_fft_factor(f->n, &f->radices, &f->npass)) return -2;
+  const size_t esz = fp64 ? 16 : 8;
+  const int n = f->n;
+  // the longest line: its buffers (none for one pass, one for two, two for
+  // more) and 24 B within kLdsBudget
+  const int nbuf = f->npass >= 3 ? 2 : (f->npass == 2 ? 1 : 0);
+  if ((size_t)nbuf * pnh_fft_lds_line(n) * esz + 24 > kLdsBudget) {
+    pnh_set_error("FFT length %d exceeds the LDS-resident limit", n);
+    return -2;
+  }
+  const int64_t n_lines = n_outer * n_inner;
+  f->inner_major = n_inner >= 8;
+  f->ct = compiled && pnh_fft_has_ct(n) && n_lines < (1LL << 32);
+  f->lines_per_block = 1;
+  const size_t tw_bytes = (size_t)n * esz;
+  const size_t line_bytes = pnh_fft_lds_bytes(*f, fp64) - tw_bytes;
+  int lg = 4;
+  while (lg > 0 && ((line_bytes << lg) + tw_bytes > kLdsBudget ||
+                    (f->ct && pnh_fft_first_pass(n) << lg > 512)))
+    --lg;
+  // fewer lines a workgroup until the launch has two workgroups per CU; along
+  // a strided axis four lines (32-byte runs) at least
+  const int lmin = f->inner_major ? 2 : 0;
+  while (lg > lmin && (n_lines >> lg) < 512) --lg;
+  // a compiled kernel's workgroup stays within one outer line: few inner
+  // lines (coils along the last axis) take the size that fills it best
+  if (f->ct && f->inner_major && n_inner < 64) {
+    int best = lg;
+    int64_t idle = 64;                     // lines idle per outer line
+    for (int g = lg; g >= 2; --g) {
+      const int64_t w = ((n_inner + (1 << g) - 1) >> g << g) - n_inner;
+      if (w < idle) { idle = w; best = g; }
+    }
+    lg = best;
+  }
+  f->lg_lines = lg;
+  f->lines_per_block = 1 << lg;
+  f->blocks_inner = (uint32_t)((n_inner + (1 << lg) - 1) >> lg);
+  f->n_blocks = f->ct && f->inner_major ? f->blocks_inner * n_outer
+                                        : (n_lines + (1 << lg) - 1) >> lg;
+  pnh_fft_magic(f->blocks_inner, &f->mul_blocks, &f->sh_blocks);
+  pnh_fft_magic((uint32_t)n_inner, &f->mul_inner, &f->sh_inner);
+  pnh_fft_magic((uint32_t)f->o_split, &f->mul_split, &f->sh_split);
+  f->threads = pnh_fft_threads(*f);
+  f->lds = (uint32_t)pnh_fft_lds_bytes(*f, fp64);
+  return 0;
+}
+
+// The line-FFT descriptor for axis `a`.
 //  forward: reads N_a valid inputs (rest zero), writes K_a outputs;
 //  inverse: reads K_a, writes the first N_a.
 //  src_image / dst_image: that side is the Nd x nb image instead of the grid.
 //  sn_side: 0 none, 1 multiply on load, 2 multiply on store.
+//  compiled: as pass_geometry (false builds the geometry anew).
 int build_pass(const pnh_plan* p, int a, bool inverse, bool src_image,
-               bool dst_image, int sn_side, int fp64, double scale, FftDesc* f) {
-  memset(f, 0, sizeof(*f));
+               bool dst_image, int sn_side, int fp64, double scale, FftDesc* f,
+               bool compiled = true) {
+  if (compiled && p->fft[fp64][inverse][a].n) {
+    *f = p->fft[fp64][inverse][a];
+  } else {
+    const int rc = pass_geometry(p, a, inverse, fp64, f, compiled);
+    if (rc) return rc;
+  }
+  f->scale = scale;
   const int D = p->D, nb = p->nb;
   int64_t kst[PNH_MAXD], nst[PNH_MAXD], sst[PNH_MAXD];
   int64_t sk = nb, sn_ = nb, ss = 1;
@@ -99,19 +177,6 @@ int build_pass(const pnh_plan* p, int a, bool inverse, bool src_image,
     nst[d] = sn_; sn_ *= p->N[d];
     sst[d] = ss; ss *= p->N[d];
   }
-  f->n = (int)p->K[a];
-  f->n_in = inverse ? (int)p->K[a] : (int)p->N[a];
-  f->n_out = inverse ? (int)p->N[a] : (int)p->K[a];
-  f->sign = inverse ? 1 : -1;
-  f->scale = scale;
-  // outer dims: d < a with image extents
-  int64_t n_outer = 1;
-  for (int d = 0; d < a; ++d) n_outer *= p->N[d];
-  f->n_outer = n_outer;
-  f->o_split = (a >= 2) ? p->N[1] : 1;
-  int64_t n_inner = nb;
-  for (int d = a + 1; d < D; ++d) n_inner *= p->K[d];
-  f->n_inner = n_inner;
   const int64_t* s_st = src_image ? nst : kst;
   const int64_t* d_st = dst_image ? nst : kst;
   f->src.t_stride = s_st[a];
@@ -131,36 +196,6 @@ int build_pass(const pnh_plan* p, int a, bool inverse, bool src_image,
   f->sn_o_stride[0] = a >= 1 ? sst[0] : 0;
   f->sn_o_stride[1] = a >= 2 ? sst[1] : 0;
   f->sn_t_stride = sst[a];
-  if (pnh_fft_factor(f->n, f->radix, f->ns, &f->npass)) return -2;
-  const size_t esz = fp64 ? 16 : 8;
-  const int n = f->n;
-  // LDS per line: line buffers (none for one pass, one for two, two for
-  // more) plus 24 B of per-line offsets
-  const int nbuf = f->npass >= 3 ? 2 : (f->npass == 2 ? 1 : 0);
-  const size_t line_bytes = (size_t)nbuf * pnh_fft_lds_line(n) * esz + 24;
-  if (line_bytes > kLdsBudget) {
-    pnh_set_error("FFT length %d exceeds the LDS-resident limit", n);
-    return -2;
-  }
-  const int64_t n_lines = n_outer * n_inner;
-  int LB;
-  if (n_inner >= 8) {
-    f->inner_major = 1;
-    LB = 16;
-    while (LB > 1 && (size_t)LB * line_bytes > kLdsBudget) LB >>= 1;
-  } else {
-    f->inner_major = 0;
-    LB = (int)(kLdsBudget / line_bytes);
-    if (LB > 16) LB = 16;
-    if (LB < 1) LB = 1;
-    // keep at least ~1024 workgroups when the lines allow it
-    while (LB > 1 && (n_lines + LB - 1) / LB < 1024) LB >>= 1;
-  }
-  f->lines_per_block = LB;
-  int rmin = f->radix[0];
-  for (int q = 1; q < f->npass; ++q) rmin = f->radix[q] < rmin ? f->radix[q] : rmin;
-  const int64_t work = (int64_t)LB * n / rmin;     // butterflies of the widest pass
-  f->threads = work >= 256 ? 256 : (work >= 128 ? 128 : 64);
   return 0;
 }
 
@@ -284,8 +319,9 @@ int plan_init(const pnh_plan_desc& d, pnh_plan* p) {
     }
     pad_cells *= p->bins.pad[a];
     n_tiles *= tg;
-    int radix[PNH_FFT_MAX_PASS], ns[PNH_FFT_MAX_PASS], np;
-    if (pnh_fft_factor((int)d.Kd[a], radix, ns, &np)) return -2;
+    uint64_t radices;
+    int np;
+    if (pnh_fft_factor((int)d.Kd[a], &radices, &np)) return -2;
     REQUIRE(d.tw_c64[a], "tw_c64[%d] missing", a);
   }
   REQUIRE(p->Ktot < (1LL << 31), "grids of 2^31 or more cells are not supported");
@@ -339,6 +375,10 @@ int plan_init(const pnh_plan_desc& d, pnh_plan* p) {
     REQUIRE(d.u_c128 && d.sn_f64, "fp64_ops needs u_c128 and sn_f64");
     for (int a = 0; a < p->D; ++a) REQUIRE(d.tw_c128[a], "fp64_ops needs tw_c128[%d]", a);
   }
+  for (int fp64 = 0; fp64 < 2; ++fp64)
+    for (int inv = 0; inv < 2; ++inv)
+      for (int a = 0; a < p->D; ++a)
+        if (pass_geometry(p, a, inv, fp64, &p->fft[fp64][inv][a])) p->fft[fp64][inv][a].n = 0;
   return 0;
 }
 
@@ -1346,7 +1386,6 @@ struct pnh_batch {
   BatchTable gather_t;                 // one block per tile
   BatchTable fft_t[3][PNH_MAXD];       // [kind][axis]
   size_t fft_lds[3][PNH_MAXD];
-  int fft_pow2[3][PNH_MAXD];
   BatchTable vec_t[3];                 // [0] grid cells, [1] samples, [2] image
   int64_t vec_chunk;
   size_t table_bytes;
@@ -1442,10 +1481,12 @@ int build_batch(const pnh_plan_desc* descs, int n, void* table, hipStream_t stre
     q.n_grid = p.Ktot;
     q.sn32 = p.d.sn_f32;
     for (int a = 0; a < D; ++a) {
-      int rc = build_pass(&p, a, false, a == D - 1, false, a == D - 1 ? 1 : 0, 0, 1.0, &q.fwd[a]);
+      int rc = build_pass(&p, a, false, a == D - 1, false, a == D - 1 ? 1 : 0, 0, 1.0, &q.fwd[a],
+                          false);
       const double sc = a == D - 1 ? 1.0 / (double)p.Ktot : 1.0;
-      if (!rc) rc = build_pass(&p, a, true, false, a == D - 1, a == D - 1 ? 2 : 0, 0, sc, &q.inv[a]);
-      if (!rc) rc = build_pass(&p, a, true, false, a == D - 1, 0, 1, sc, &q.inv64[a]);
+      if (!rc) rc = build_pass(&p, a, true, false, a == D - 1, a == D - 1 ? 2 : 0, 0, sc, &q.inv[a],
+                               false);
+      if (!rc) rc = build_pass(&p, a, true, false, a == D - 1, 0, 1, sc, &q.inv64[a], false);
       if (rc) return rc;
       q.tw32[a] = p.d.tw_c64[a];
       q.tw64[a] = p.d.tw_c128[a];
@@ -1468,19 +1509,15 @@ int build_batch(const pnh_plan_desc* descs, int n, void* table, hipStream_t stre
     for (int a = 0; a < D; ++a) {
       std::vector<int64_t> nbk(n);
       size_t lds = 0;
-      int pow2 = 1;
       for (int i = 0; i < n; ++i) {
         FftDesc& f = kind == BFFT_FWD ? probs[i].fwd[a]
                                       : (kind == BFFT_INV ? probs[i].inv[a] : probs[i].inv64[a]);
         const int64_t lines = f.n_outer * f.n_inner;
-        nbk[i] = (lines + f.lines_per_block - 1) / f.lines_per_block;
-        lds = std::max(lds, pnh_fft_lds_bytes(f, kind == BFFT_INV64));
-        for (int q = 0; q < f.npass; ++q)
-          pow2 &= (f.radix[q] == 2 || f.radix[q] == 4 || f.radix[q] == 8 || f.radix[q] == 16);
+        nbk[i] = (lines + f.lines_per_block - 1) / f.lines_per_block;   // as fft_batch_kernel
+        lds = std::max(lds, (size_t)f.lds);
       }
       add_table(blob, nbk, &of_tab[kind][a], &of_first[kind][a], &b->fft_t[kind][a].n_blocks);
       b->fft_lds[kind][a] = lds;
-      b->fft_pow2[kind][a] = pow2;
     }
   // vector tables: grid cells, samples, image
   size_t ov_tab[3], ov_first[3];
@@ -1548,7 +1585,7 @@ int batch_passes(const pnh_batch* b, int kind, int fp64, const void* image_in,
     const bool img_in = kind == BFFT_FWD && a == b->D - 1;
     const bool img_out = kind != BFFT_FWD && a == b->D - 1;
     int rc = pnh_batch_fft_launch(b->probs, b->fft_t[kind][a], a, kind, fp64,
-                                  b->fft_pow2[kind][a], b->fft_lds[kind][a], b->fft_threads,
+                                  b->fft_lds[kind][a], b->fft_threads,
                                   img_in ? image_in : grid, img_in, img_out ? image_out : grid,
                                   img_out, done, all_done, s);
     if (rc) return rc;

@@ -71,7 +71,7 @@ int pnh_batch_y2k_launch(const BatchProblem* probs, const int2* items, int64_t n
                          int64_t pad_cells, int threads, const void* y, void* k, void* part,
                          const int* done, const int* all_done, hipStream_t s);
 int pnh_batch_fft_launch(const BatchProblem* probs, const BatchTable& t, int axis,
-                         int kind, int fp64, int pow2, size_t lds, int threads,
+                         int kind, int fp64, size_t lds, int threads,
                          const void* in, int in_image, void* out, int out_image,
                          const int* done, const int* all_done, hipStream_t s);
 // One element-wise / CG step over every problem's packed vector (op

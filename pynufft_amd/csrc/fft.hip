@@ -1,169 +1,21 @@
 // LDS-resident Stockham FFT over lines of a strided N-d array (gfx950).
 //
-// One launch transforms every line along one axis.  A workgroup loads LB lines
-// into LDS (zero-filling past n_in, so zero-padding is fused), runs all radix
-// passes in LDS (ping-pong buffers, radices 8/4/2/3/5 and a generic small odd
-// radix), and writes the first n_out outputs of each line (so cropping is
-// fused).  The real apodization factor sn and a scalar may be applied on the
-// load side (forward: x2xx fused) or on the store side (adjoint: xx2x fused).
+// One launch transforms every line along one axis.  A workgroup takes LB
+// lines: the first radix pass reads global memory (zero-filling past n_in, so
+// zero-padding is fused, and applying the real apodization factor sn:
+// x2xx fused), the passes exchange through LDS, and the last one writes the
+// first n_out outputs of each line (cropping, the scale and xx2x fused).
 //
 // Semantics follow numpy.fft: the forward kernel is exp(-2 pi i t/n), the
-// inverse exp(+2 pi i t/n) with the 1/n factors folded into `scale`.
-#include "common.h"
-#include "fft.h"
+// inverse exp(+2 pi i t/n) with the 1/n factors folded into `scale`.  The
+// butterflies are forward only: the inverse is conj(F(conj(x))), the
+// conjugations riding on the load and the final scale.
+//
+// The lengths that plans use have kernels compiled for them (fft_ct.h);
+// fft_lines_kernel below takes every other length, and the batches.
+#include "fft_ct.h"
 
 namespace {
-
-template <typename C, typename T>
-__device__ __forceinline__ C mul_neg_i(C a, int sign) {
-  // multiply by (sign * i): sign=-1 -> -i, sign=+1 -> +i
-  C z;
-  if (sign < 0) { z.x = a.y; z.y = -a.x; } else { z.x = -a.y; z.y = a.x; }
-  return z;
-}
-
-template <typename T>
-__device__ __forceinline__ void dft2(typename cplx<T>::t* v) {
-  typename cplx<T>::t a = v[0], b = v[1];
-  v[0] = cadd(a, b); v[1] = csub(a, b);
-}
-
-template <typename T>
-__device__ __forceinline__ void dft4(typename cplx<T>::t* v, int sign) {
-  typedef typename cplx<T>::t C;
-  C t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]);
-  C t2 = cadd(v[1], v[3]), t3 = csub(v[1], v[3]);
-  C t3r = mul_neg_i<C, T>(t3, sign);  // sign*i*(v1-v3)
-  v[0] = cadd(t0, t2);
-  v[2] = csub(t0, t2);
-  v[1] = cadd(t1, t3r);
-  v[3] = csub(t1, t3r);
-}
-
-template <typename T>
-__device__ __forceinline__ void dft8(typename cplx<T>::t* v, int sign) {
-  typedef typename cplx<T>::t C;
-  const T h = (T)0.70710678118654752440;
-  // even/odd split: E = DFT4(v0,v2,v4,v6), O = DFT4(v1,v3,v5,v7)
-  C e[4] = {v[0], v[2], v[4], v[6]};
-  C o[4] = {v[1], v[3], v[5], v[7]};
-  dft4<T>(e, sign);
-  dft4<T>(o, sign);
-  // twiddles w8^q = exp(sign*2*pi*i*q/8), q = 0..3
-  C o1, o2, o3;
-  T s = (T)sign;
-  // q=1: (1 + s i) h
-  o1.x = (o[1].x - s * o[1].y) * h;
-  o1.y = (o[1].y + s * o[1].x) * h;
-  // q=2: s i
-  o2 = mul_neg_i<C, T>(o[2], sign);
-  // q=3: (-1 + s i) h
-  o3.x = (-o[3].x - s * o[3].y) * h;
-  o3.y = (-o[3].y + s * o[3].x) * h;
-  v[0] = cadd(e[0], o[0]); v[4] = csub(e[0], o[0]);
-  v[1] = cadd(e[1], o1);   v[5] = csub(e[1], o1);
-  v[2] = cadd(e[2], o2);   v[6] = csub(e[2], o2);
-  v[3] = cadd(e[3], o3);   v[7] = csub(e[3], o3);
-}
-
-// 16-point DFT as 4 x 4: DFTs over n1 of x[4 n1 + n2], twiddles
-// W16^(n2 k1), DFTs over n2; W = exp(sign 2 pi i / 16).
-template <typename T>
-__device__ __forceinline__ void dft16(typename cplx<T>::t* v, int sign) {
-  typedef typename cplx<T>::t C;
-  const T c1 = (T)0.92387953251128675613, s1 = (T)0.38268343236508977173;
-  const T h = (T)0.70710678118654752440;
-  const T sg = (T)sign;
-  C a[4][4];
-#pragma unroll
-  for (int n2 = 0; n2 < 4; ++n2) {
-    C t[4] = {v[n2], v[n2 + 4], v[n2 + 8], v[n2 + 12]};
-    dft4<T>(t, sign);
-#pragma unroll
-    for (int k1 = 0; k1 < 4; ++k1) a[n2][k1] = t[k1];
-  }
-  // W16^e for e = n2 * k1 in {1, 2, 3, 4, 6, 9}
-  const C w1 = mk<T>(c1, sg * s1), w2 = mk<T>(h, sg * h), w3 = mk<T>(s1, sg * c1);
-  const C w4 = mk<T>((T)0, sg), w6 = mk<T>(-h, sg * h), w9 = mk<T>(-c1, -sg * s1);
-  a[1][1] = cmul(a[1][1], w1); a[1][2] = cmul(a[1][2], w2); a[1][3] = cmul(a[1][3], w3);
-  a[2][1] = cmul(a[2][1], w2); a[2][2] = cmul(a[2][2], w4); a[2][3] = cmul(a[2][3], w6);
-  a[3][1] = cmul(a[3][1], w3); a[3][2] = cmul(a[3][2], w6); a[3][3] = cmul(a[3][3], w9);
-#pragma unroll
-  for (int k1 = 0; k1 < 4; ++k1) {
-    C t[4] = {a[0][k1], a[1][k1], a[2][k1], a[3][k1]};
-    dft4<T>(t, sign);
-#pragma unroll
-    for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = t[k2];
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ void dft3(typename cplx<T>::t* v, int sign) {
-  typedef typename cplx<T>::t C;
-  const T c = (T)-0.5, s = (T)0.86602540378443864676 * (T)sign;
-  C t1 = cadd(v[1], v[2]);
-  C t2 = csub(v[1], v[2]);
-  C m = cadd(v[0], cscale(t1, c));
-  // s*i*t2
-  C r; r.x = -s * t2.y; r.y = s * t2.x;
-  v[0] = cadd(v[0], t1);
-  v[1] = cadd(m, r);
-  v[2] = csub(m, r);
-}
-
-template <typename T>
-__device__ __forceinline__ void dft5(typename cplx<T>::t* v, int sign) {
-  typedef typename cplx<T>::t C;
-  const T c1 = (T)0.30901699437494742410, c2 = (T)-0.80901699437494742410;
-  const T s1 = (T)0.95105651629515357212 * (T)sign;
-  const T s2 = (T)0.58778525229247312917 * (T)sign;
-  C a1 = cadd(v[1], v[4]), b1 = csub(v[1], v[4]);
-  C a2 = cadd(v[2], v[3]), b2 = csub(v[2], v[3]);
-  C m1 = cadd(v[0], cadd(cscale(a1, c1), cscale(a2, c2)));
-  C m2 = cadd(v[0], cadd(cscale(a1, c2), cscale(a2, c1)));
-  // i*(s1 b1 + s2 b2), i*(s2 b1 - s1 b2)
-  C n1 = cadd(cscale(b1, s1), cscale(b2, s2));
-  C n2 = csub(cscale(b1, s2), cscale(b2, s1));
-  C r1; r1.x = -n1.y; r1.y = n1.x;
-  C r2; r2.x = -n2.y; r2.y = n2.x;
-  v[0] = cadd(v[0], cadd(a1, a2));
-  v[1] = cadd(m1, r1); v[4] = csub(m1, r1);
-  v[2] = cadd(m2, r2); v[3] = csub(m2, r2);
-}
-
-// Generic small odd radix R via the length-n twiddle table: w_R^k = tw[k*(n/R)].
-template <typename T, int R>
-__device__ __forceinline__ void dftg(typename cplx<T>::t* v, int n,
-                                     const typename cplx<T>::t* tw, int sign) {
-  typedef typename cplx<T>::t C;
-  C out[R];
-  const int step = n / R;
-#pragma unroll
-  for (int q = 0; q < R; ++q) {
-    C acc = v[0];
-#pragma unroll
-    for (int r = 1; r < R; ++r) {
-      C w = tw[((r * q) % R) * step];
-      if (sign > 0) w.y = -w.y;
-      acc = cadd(acc, cmul(v[r], w));
-    }
-    out[q] = acc;
-  }
-#pragma unroll
-  for (int q = 0; q < R; ++q) v[q] = out[q];
-}
-
-template <typename T, int R>
-__device__ __forceinline__ void dft_r(typename cplx<T>::t* v, int n,
-                                      const typename cplx<T>::t* tw, int sign) {
-  if (R == 2) dft2<T>(v);
-  else if (R == 3) dft3<T>(v, sign);
-  else if (R == 4) dft4<T>(v, sign);
-  else if (R == 5) dft5<T>(v, sign);
-  else if (R == 8) dft8<T>(v, sign);
-  else if (R == 16) dft16<T>(v, sign);
-  else dftg<T, R>(v, n, tw, sign);
-}
 
 // q = i / n and r = i % n for 0 <= i < 2^22 and 1 <= n, with rcp = 1.0f / n
 // (the float estimate is off by at most one; one correction step fixes it)
@@ -175,264 +27,276 @@ __device__ __forceinline__ int fdivmod(int i, int n, float rcp, int& r) {
   return q;
 }
 
-// i / n, i % n: shifts for powers of two, else the float reciprocal
-template <bool POW2>
-__device__ __forceinline__ int divmod_n(int i, int n, int log2n, float rcp, int& r) {
-  if (POW2) { r = i & (n - 1); return i >> log2n; }
-  return fdivmod(i, n, rcp, r);
-}
-
-// One Stockham radix-R pass over LB lines.  Butterfly (l, j), j < n/R,
-// reads in(l, j + r n/R) for r < R, applies the twiddles of a stage after
-// ns points, and writes out(l, (j / ns) ns R + j % ns + r ns).  With
-// lines_fast, consecutive threads take consecutive lines (coalesced global
-// access along a strided axis); else consecutive j.
-template <typename T, int R, bool POW2, typename LD, typename ST>
-__device__ __forceinline__ void stockham_pass(int n, int LB, int ns, bool lines_fast,
-                                              const typename cplx<T>::t* tw, int sign,
-                                              int tid, int nthr, LD load, ST store) {
+// One Stockham radix-R pass over LB lines in LDS.  Butterfly (l, j), j <
+// n/R, reads points j + r n/R for r < R, applies the twiddles of a stage
+// after ns points, and writes points (j / ns) ns R + j % ns + r ns.
+template <typename T, int R>
+__device__ __forceinline__ void stockham_pass(int n, int LB, int ns, int ld,
+                                              const typename cplx<T>::t* tw,
+                                              const typename cplx<T>::t* src,
+                                              typename cplx<T>::t* dst) {
   typedef typename cplx<T>::t C;
   const int nb = n / R;
   const int twstep = n / (ns * R);
   const int total = LB * nb;
-  const int lg_nb = POW2 ? __builtin_ctz(nb) : 0;
-  const int lg_ns = POW2 ? __builtin_ctz(ns) : 0;
-  const bool lb_pow2 = (LB & (LB - 1)) == 0;
-  const int lg_lb = lb_pow2 ? __builtin_ctz(LB) : 0;
-  const float r_nb = 1.0f / (float)nb, r_ns = 1.0f / (float)ns, r_lb = 1.0f / (float)LB;
-  for (int idx = tid; idx < total; idx += nthr) {
-    int l, j, k;
-    if (lines_fast) {
-      if (lb_pow2) { l = idx & (LB - 1); j = idx >> lg_lb; }
-      else j = fdivmod(idx, LB, r_lb, l);
-    } else {
-      l = divmod_n<POW2>(idx, nb, lg_nb, r_nb, j);
-    }
-    const int jq = divmod_n<POW2>(j, ns, lg_ns, r_ns, k);
+  const float r_nb = 1.0f / (float)nb, r_ns = 1.0f / (float)ns;
+  for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
+    int j, k;
+    const int l = fdivmod(idx, nb, r_nb, j);
+    const int jq = fdivmod(j, ns, r_ns, k);
+    const int kt = k * twstep;
     C v[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = load(l, j + r * nb);
-    if (ns > 1) {
-#pragma unroll
-      for (int r = 1; r < R; ++r) {
-        C w = tw[r * k * twstep];
-        if (sign > 0) w.y = -w.y;
-        v[r] = cmul(v[r], w);
-      }
+    for (int r = 0; r < R; ++r) {
+      const int t = j + r * nb;
+      v[r] = src[l * ld + t + (t >> 4)];
     }
-    dft_r<T, R>(v, n, tw, sign);
+#pragma unroll
+    for (int r = 1; r < R; ++r) v[r] = cmul_fma(v[r], tw[r * kt]);
+    Dft<T, R>::run(v);
     const int o = jq * ns * R + k;
 #pragma unroll
-    for (int r = 0; r < R; ++r) store(l, o + r * ns, v[r]);
+    for (int r = 0; r < R; ++r) {
+      const int t = o + r * ns;
+      dst[l * ld + t + (t >> 4)] = v[r];
+    }
   }
 }
 
-template <typename T, bool POW2, typename LD, typename ST>
-__device__ __forceinline__ void run_pass(int R, int n, int LB, int ns, bool lines_fast,
-                                         const typename cplx<T>::t* tw, int sign, int tid,
-                                         int nthr, LD load, ST store) {
-  if (POW2) {
-    if (R == 16) stockham_pass<T, 16, true>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store);
-    else if (R == 8) stockham_pass<T, 8, true>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store);
-    else if (R == 4) stockham_pass<T, 4, true>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store);
-    else stockham_pass<T, 2, true>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store);
-    return;
-  }
-  switch (R) {
-    case 2: stockham_pass<T, 2, false>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store); break;
-    case 3: stockham_pass<T, 3, false>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store); break;
-    case 4: stockham_pass<T, 4, false>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store); break;
-    case 5: stockham_pass<T, 5, false>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store); break;
-    case 7: stockham_pass<T, 7, false>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store); break;
-    case 8: stockham_pass<T, 8, false>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store); break;
-    case 11: stockham_pass<T, 11, false>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store); break;
-    case 13: stockham_pass<T, 13, false>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store); break;
-    default: stockham_pass<T, 16, false>(n, LB, ns, lines_fast, tw, sign, tid, nthr, load, store); break;
-  }
-}
-
+// Any length of radices 2 to 16 (run-time schedule).  The lines are copied
+// into LDS, transformed there between two buffers, and copied out, so the
+// radix switch appears once (with it at the global ends too the kernel was
+// 240 KB of code).  in_ and out_ may alias (in-place passes): a workgroup
+// reads all its lines before its first store, and other workgroups own other
+// lines.  LDS: the twiddle table, then two line buffers of
+// LB x pnh_fft_lds_stride(n).
 template <typename T>
-__device__ __forceinline__ T ld_sn(const void* p, int64_t i) {
-  return (T)((const T*)p)[i];
-}
-
-// Offsets of line `l` (flattened over outer x inner) in a buffer.
-__device__ __forceinline__ int64_t line_base(const FftSide& s, int64_t o0,
-                                             int64_t o1, int64_t b) {
-  return o0 * s.o_stride[0] + o1 * s.o_stride[1] + b * s.b_stride;
-}
-
-// POW2: every radix is 2, 4, 8 or 16 (shift/mask indexing).  The first
-// pass reads its inputs from global memory (zero padding and load-side
-// apodization fused) and the last pass writes its outputs there (crop,
-// scale and store-side apodization fused); the passes in between go through
-// LDS.  in_ and out_ may alias (in-place passes): a workgroup reads all its
-// lines before its first store, and other workgroups own other lines.
-// LDS: one line buffer (two with three or more passes), lines of
-// n + n/16 + 1 elements (one pad element per 16 against bank conflicts),
-// then per-line source/destination/apodization offsets.
-template <typename T, bool POW2>
 __device__ __forceinline__ void fft_body(const FftDesc& d, const void* in_, void* out_,
                                          const void* __restrict__ tw_, int64_t blk,
                                          unsigned char* smem_raw) {
   typedef typename cplx<T>::t C;
-  const int n = d.n;
-  const int LB = d.lines_per_block;
-  const int ld = pnh_fft_lds_line(n);
-  const int nbuf = d.npass >= 3 ? 2 : (d.npass == 2 ? 1 : 0);
-  C* buf0 = reinterpret_cast<C*>(smem_raw);
-  C* buf1 = buf0 + (size_t)LB * ld;
-  int64_t* loff = reinterpret_cast<int64_t*>(buf0 + (size_t)nbuf * LB * ld);  // [3][LB]
+  const int n = d.n, LB = d.lines_per_block;
+  const int ld = pnh_fft_lds_stride(n);
+  C* tws = reinterpret_cast<C*>(smem_raw);
+  C* src = tws + n;
+  C* dst = src + (size_t)LB * ld;
   const C* in = (const C*)in_;
   C* out = (C*)out_;
   const C* __restrict__ tw = (const C*)tw_;
-
+  const int nthr = blockDim.x, tid = threadIdx.x;
   const int64_t line0 = blk * LB;
   const int64_t n_lines = d.n_outer * d.n_inner;
-  const int nthr = blockDim.x;
-  const int tid = threadIdx.x;
   const int nl = (int)(n_lines - line0 < LB ? n_lines - line0 : LB);  // lines present
-
-  if (tid < LB) {
-    const int64_t L = line0 + (tid < nl ? tid : 0);
-    const int64_t o = L / d.n_inner, b = L - o * d.n_inner;
-    const int64_t o0 = o / d.o_split, o1 = o - o0 * d.o_split;
-    loff[tid] = line_base(d.src, o0, o1, b);
-    loff[LB + tid] = line_base(d.dst, o0, o1, b);
-    loff[2 * LB + tid] = o0 * d.sn_o_stride[0] + o1 * d.sn_o_stride[1];
-  }
-  __syncthreads();
-
-  const int64_t st = d.src.t_stride, dt = d.dst.t_stride;
-  const int n_in = d.n_in, n_out = d.n_out;
-  const int sn_side = d.sn_side;
-  const T scale = (T)d.scale;
-  auto gload = [&](int l, int t) -> C {
+  const bool fast = d.inner_major != 0;
+  const float r_lb = 1.0f / (float)LB, r_n = 1.0f / (float)n;
+  const T cj = d.sign > 0 ? (T)-1 : (T)1;         // inverse: conjugate in and out
+  // source, destination and apodization offset of line l of the workgroup
+  struct Line { int64_t src, dst, sn; };
+  auto line = [&](int l) -> Line {
+    const int64_t L = line0 + l;
+    int64_t o, b, o0, o1;
+    if (n_lines < (1LL << 31)) {
+      const uint32_t ou = (uint32_t)L / (uint32_t)d.n_inner;
+      o = ou;
+      b = (uint32_t)L - ou * (uint32_t)d.n_inner;
+      const uint32_t q = ou / (uint32_t)d.o_split;
+      o0 = q;
+      o1 = ou - q * (uint32_t)d.o_split;
+    } else {
+      o = L / d.n_inner; b = L - o * d.n_inner;
+      o0 = o / d.o_split; o1 = o - o0 * d.o_split;
+    }
+    return Line{o0 * d.src.o_stride[0] + o1 * d.src.o_stride[1] + b * d.src.b_stride,
+                o0 * d.dst.o_stride[0] + o1 * d.dst.o_stride[1] + b * d.dst.b_stride,
+                o0 * d.sn_o_stride[0] + o1 * d.sn_o_stride[1]};
+  };
+  // element i of the copies: consecutive threads on consecutive lines along a
+  // strided axis, else along the line
+  auto point = [&](int i, int& t) -> int {
+    int l;
+    if (fast) t = fdivmod(i, LB, r_lb, l);
+    else l = fdivmod(i, n, r_n, t);
+    return l;
+  };
+  for (int i = tid; i < n; i += nthr) tws[i] = tw[i];
+  const int total = LB * n;
+#pragma unroll 4
+  for (int i = tid; i < total; i += nthr) {
+    int t;
+    const int l = point(i, t);
     C v = mk<T>((T)0, (T)0);
-    if (l < nl && t < n_in) {
-      v = in[loff[l] + (int64_t)t * st];
-      if (sn_side == 1) {
-        const T s = ld_sn<T>(d.sn, loff[2 * LB + l] + (int64_t)t * d.sn_t_stride);
+    if (l < nl && t < d.n_in) {
+      const Line li = line(l);
+      v = in[li.src + (int64_t)t * d.src.t_stride];
+      if (d.sn_side == 1) {
+        const T s = ((const T*)d.sn)[li.sn + (int64_t)t * d.sn_t_stride];
         v.x *= s; v.y *= s;
       }
     }
-    return v;
-  };
-  auto gstore = [&](int l, int t, C v) {
-    if (l < nl && t < n_out) {
-      T s = scale;
-      if (sn_side == 2) s *= ld_sn<T>(d.sn, loff[2 * LB + l] + (int64_t)t * d.sn_t_stride);
-      v.x *= s; v.y *= s;
-      out[loff[LB + l] + (int64_t)t * dt] = v;
-    }
-  };
-  auto at = [&](C* b, int l, int t) -> C& { return b[l * ld + t + (t >> 4)]; };
-  const int sign = d.sign;
-  const bool fast = d.inner_major != 0;
-
-  if (d.npass == 1) {
-    run_pass<T, POW2>(d.radix[0], n, LB, 1, fast, tw, sign, tid, nthr, gload, gstore);
-    return;
+    v.y *= cj;
+    src[l * ld + t + (t >> 4)] = v;
   }
-  run_pass<T, POW2>(d.radix[0], n, LB, d.ns[0], fast, tw, sign, tid, nthr, gload,
-                    [&](int l, int t, C v) { at(buf0, l, t) = v; });
-  __syncthreads();
-  C* src = buf0;
-  C* dst = buf1;
-  for (int p = 1; p + 1 < d.npass; ++p) {
-    run_pass<T, POW2>(d.radix[p], n, LB, d.ns[p], false, tw, sign, tid, nthr,
-                      [&](int l, int t) -> C { return at(src, l, t); },
-                      [&](int l, int t, C v) { at(dst, l, t) = v; });
+  int ns = 1;
+  for (int p = 0; p < d.npass; ++p) {
     __syncthreads();
+    const int R = pnh_fft_radix(d.radices, p);
+    switch (R) {
+#define PNH_R(r) case r: stockham_pass<T, r>(n, LB, ns, ld, tws, src, dst); break;
+      PNH_R(2) PNH_R(3) PNH_R(4) PNH_R(5) PNH_R(6) PNH_R(7) PNH_R(8) PNH_R(9) PNH_R(10)
+      PNH_R(11) PNH_R(12) PNH_R(13) PNH_R(14) PNH_R(15)
+      default: stockham_pass<T, 16>(n, LB, ns, ld, tws, src, dst); break;
+#undef PNH_R
+    }
+    ns *= R;
     C* tmp = src; src = dst; dst = tmp;
   }
-  const int pl = d.npass - 1;
-  run_pass<T, POW2>(d.radix[pl], n, LB, d.ns[pl], fast, tw, sign, tid, nthr,
-                    [&](int l, int t) -> C { return at(src, l, t); }, gstore);
+  __syncthreads();
+  const T scale = (T)d.scale, scale_im = scale * cj;
+  const int kept = LB * d.n_out;
+  const float r_o = 1.0f / (float)d.n_out;
+#pragma unroll 4
+  for (int i = tid; i < kept; i += nthr) {
+    int l, t;
+    if (fast) t = fdivmod(i, LB, r_lb, l);
+    else l = fdivmod(i, d.n_out, r_o, t);
+    if (l >= nl) continue;
+    const Line li = line(l);
+    C v = src[l * ld + t + (t >> 4)];
+    if (d.sn_side == 2) {
+      const T s = ((const T*)d.sn)[li.sn + (int64_t)t * d.sn_t_stride];
+      v.x *= s; v.y *= s;
+    }
+    out[li.dst + (int64_t)t * d.dst.t_stride] = mk<T>(v.x * scale, v.y * scale_im);
+  }
 }
 
-template <typename T, bool POW2>
+template <typename T>
 __global__ void __launch_bounds__(256)
 fft_lines_kernel(FftDesc d, const void* in_, void* out_,
                  const void* __restrict__ tw_, const int* __restrict__ skip) {
   if (skip && *skip) return;
   extern __shared__ unsigned char smem_raw[];
-  fft_body<T, POW2>(d, in_, out_, tw_, blockIdx.x, smem_raw);
+  fft_body<T>(d, in_, out_, tw_, xcd_unit(blockIdx.x, gridDim.x), smem_raw);
 }
 
-}  // namespace
-
-int pnh_fft_launch(const FftDesc& d, int fp64, const void* in, void* out,
-                   const void* tw, const int* skip, hipStream_t stream) {
-  const int64_t n_lines = d.n_outer * d.n_inner;
-  if (n_lines <= 0) return 0;
-  const int64_t nblk = (n_lines + d.lines_per_block - 1) / d.lines_per_block;
-  const size_t esz = fp64 ? 16 : 8;
-  const size_t lds = pnh_fft_lds_bytes(d, fp64);
-  dim3 grid((unsigned)nblk), block(d.threads);
-  bool pow2 = true;
-  for (int p = 0; p < d.npass; ++p)
-    pow2 = pow2 && (d.radix[p] == 2 || d.radix[p] == 4 || d.radix[p] == 8 || d.radix[p] == 16);
-  if (fp64) {
-    if (pow2)
-      hipLaunchKernelGGL((fft_lines_kernel<double, true>), grid, block, lds, stream, d,
-                         in, out, tw, skip);
-    else
-      hipLaunchKernelGGL((fft_lines_kernel<double, false>), grid, block, lds, stream, d,
-                         in, out, tw, skip);
-  } else {
-    if (pow2)
-      hipLaunchKernelGGL((fft_lines_kernel<float, true>), grid, block, lds, stream, d,
-                         in, out, tw, skip);
-    else
-      hipLaunchKernelGGL((fft_lines_kernel<float, false>), grid, block, lds, stream, d,
-                         in, out, tw, skip);
-  }
+template <typename T>
+int launch_lines(const FftDesc& d, const void* in, void* out, const void* tw, const int* skip,
+                 hipStream_t stream) {
+  auto kern = fft_lines_kernel<T>;
+  pnh_fft_allow_lds((const void*)kern, d.lds);
+  hipLaunchKernelGGL(kern, dim3((unsigned)d.n_blocks), dim3(d.threads), d.lds, stream, d, in, out,
+                     tw, skip);
   PNH_LAUNCH_CHECK();
   return 0;
 }
 
-size_t pnh_fft_lds_bytes(const FftDesc& d, int fp64) {
-  const size_t esz = fp64 ? 16 : 8;
-  const int nbuf = d.npass >= 3 ? 2 : (d.npass == 2 ? 1 : 0);
-  return (size_t)nbuf * d.lines_per_block * pnh_fft_lds_line(d.n) * esz +
-         3 * (size_t)d.lines_per_block * sizeof(int64_t);
+}  // namespace
+
+#define PNH_CT_DECL(p) \
+  int pnh_fft_ct_part##p(const FftDesc&, int, const void*, void*, const void*, const int*, \
+                         hipStream_t);
+PNH_CT_DECL(0) PNH_CT_DECL(1) PNH_CT_DECL(2) PNH_CT_DECL(3) PNH_CT_DECL(4) PNH_CT_DECL(5)
+PNH_CT_DECL(6)
+#undef PNH_CT_DECL
+
+bool pnh_fft_has_ct(int n) {
+  return n >= PNH_CT_MIN && n <= PNH_CT_MAX && n % 2 == 0 && radices_of(n).r[0] > 0;
 }
 
-// Factor n into radices: 16 first, then 8, 4, 2, then 3, 5, then the other
-// small odd primes.
-int pnh_fft_factor(int n, int* radix, int* ns, int* npass) {
-  int m = n, cnt = 0;
-  int prod = 1;
-  while (m > 1) {
-    int R;
-    if (m % 16 == 0) R = 16;
-    else if (m % 8 == 0) R = 8;
-    else if (m % 4 == 0) R = 4;
-    else if (m % 2 == 0) R = 2;
-    else if (m % 3 == 0) R = 3;
-    else if (m % 5 == 0) R = 5;
-    else {
-      R = 0;
-      const int generic[3] = {7, 11, 13};
-      for (int q = 0; q < 3; ++q)
-        if (m % generic[q] == 0) { R = generic[q]; break; }
-      if (R == 0) {
-        pnh_set_error("FFT length %d has a prime factor other than 2, 3, 5, 7, 11, 13", n);
-        return -1;
-      }
+int pnh_fft_launch(const FftDesc& d, int fp64, const void* in, void* out,
+                   const void* tw, const int* skip, hipStream_t stream) {
+  if (d.n_outer * d.n_inner <= 0) return 0;
+  if (d.ct) {
+    switch ((d.n - PNH_CT_MIN) / 2 % PNH_CT_PARTS) {
+      case 0: return pnh_fft_ct_part0(d, fp64, in, out, tw, skip, stream);
+      case 1: return pnh_fft_ct_part1(d, fp64, in, out, tw, skip, stream);
+      case 2: return pnh_fft_ct_part2(d, fp64, in, out, tw, skip, stream);
+      case 3: return pnh_fft_ct_part3(d, fp64, in, out, tw, skip, stream);
+      case 4: return pnh_fft_ct_part4(d, fp64, in, out, tw, skip, stream);
+      case 5: return pnh_fft_ct_part5(d, fp64, in, out, tw, skip, stream);
+      default: return pnh_fft_ct_part6(d, fp64, in, out, tw, skip, stream);
     }
-    if (cnt >= PNH_FFT_MAX_PASS) {
-      pnh_set_error("FFT length %d needs too many passes", n);
-      return -1;
-    }
-    radix[cnt] = R;
-    ns[cnt] = prod;
-    prod *= R;
-    m /= R;
-    ++cnt;
   }
-  *npass = cnt;
+  return fp64 ? launch_lines<double>(d, in, out, tw, skip, stream)
+              : launch_lines<float>(d, in, out, tw, skip, stream);
+}
+
+void pnh_fft_magic(uint32_t d, uint32_t* mul, int* shift) {
+  int L = 0;
+  while (L < 32 && (1ULL << L) < d) ++L;        // ceil(log2 d)
+  if ((1ULL << L) == d) { *mul = 0; *shift = L; return; }
+  *mul = (uint32_t)((((1ULL << L) - d) << 32) / d + 1);
+  *shift = L - 1;
+}
+
+int pnh_fft_first_pass(int n) { return n / radices_of(n).r[0]; }
+
+int pnh_fft_threads(const FftDesc& d) {
+  if (!d.ct) return 256;
+  const Radices rs = radices_of(d.n);
+  const int rl = rs.r[2] > 1 ? rs.r[2] : rs.r[1];
+  // one butterfly per thread in the first pass; in the others one per thread
+  // up to 256 threads, or 512 where the workgroups are too few to fill the
+  // chip (390 x 462 per transform 9.4 us at 256, 8.9 at 512; 256^3 66.5 at
+  // 256, 70.7 at 512)
+  const int first = d.n / rs.r[0] << d.lg_lines, most = d.n / rl << d.lg_lines;
+  const int cap = d.n_blocks < 512 ? 512 : 256;
+  const int want = first > cap ? first : (most < cap ? most : cap);
+  return (want + 63) / 64 * 64;
+}
+
+size_t pnh_fft_lds_bytes(const FftDesc& d, int fp64) {
+  const size_t esz = fp64 ? 16 : 8;
+  const int nbuf = d.ct && radices_of(d.n).r[2] == 1 ? 1 : 2;
+  return ((size_t)nbuf * d.lines_per_block * pnh_fft_lds_stride(d.n) + d.n) * esz;
+}
+
+// Dynamic LDS above 64 KB must be allowed per kernel before the launch.
+void pnh_fft_allow_lds(const void* kernel, size_t bytes) {
+  if (bytes > 65536)
+    (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
+// Radices of n (each 2 to 16): the fewest passes, then the smallest sum of
+// radices (the least work and the most threads per line), in falling order.
+// n <= 4096 in every accepted plan, so three passes usually do.
+static void best_radices(int m, int max_r, int left, int* cur, int depth, int sum, int* best,
+                         int* best_np, int* best_sum) {
+  if (m == 1) {
+    if (depth < *best_np || (depth == *best_np && sum < *best_sum)) {
+      *best_np = depth;
+      *best_sum = sum;
+      for (int i = 0; i < depth; ++i) best[i] = cur[i];
+    }
+    return;
+  }
+  if (depth >= left || depth >= *best_np) return;
+  for (int r = max_r; r >= 2; --r)
+    if (m % r == 0) {
+      cur[depth] = r;
+      best_radices(m / r, r, left, cur, depth + 1, sum + r, best, best_np, best_sum);
+    }
+}
+
+int pnh_fft_factor(int n, uint64_t* radices, int* npass) {
+  int m = n;
+  const int primes[6] = {2, 3, 5, 7, 11, 13};
+  for (int q = 0; q < 6; ++q)
+    while (m % primes[q] == 0 && m > 1) m /= primes[q];
+  if (m != 1) {
+    pnh_set_error("FFT length %d has a prime factor other than 2, 3, 5, 7, 11, 13", n);
+    return -1;
+  }
+  int cur[PNH_FFT_MAX_PASS], best[PNH_FFT_MAX_PASS];
+  int np = PNH_FFT_MAX_PASS + 1, sum = 0;
+  best_radices(n, 16, PNH_FFT_MAX_PASS, cur, 0, 0, best, &np, &sum);
+  if (np > PNH_FFT_MAX_PASS) {
+    pnh_set_error("FFT length %d needs too many passes", n);
+    return -1;
+  }
+  *radices = 0;
+  for (int p = 0; p < np; ++p) *radices |= (uint64_t)(best[p] - 1) << (4 * p);
+  *npass = np;
   return 0;
 }
 
@@ -441,7 +305,7 @@ int pnh_fft_factor(int n, int* radix, int* ns, int* npass) {
 
 namespace {
 
-template <typename T, bool POW2>
+template <typename T>
 __global__ void __launch_bounds__(256)
 fft_batch_kernel(const BatchProblem* __restrict__ probs, BatchTable t, int axis, int kind,
                  const void* in_, int in_image, void* out_, int out_image,
@@ -460,24 +324,22 @@ fft_batch_kernel(const BatchProblem* __restrict__ probs, BatchTable t, int axis,
   const void* tw = kind == BFFT_INV64 ? pr.tw64[axis] : pr.tw32[axis];
   const C* in = (const C*)in_ + (in_image ? pr.x_off : pr.k_off);
   C* out = (C*)out_ + (out_image ? pr.x_off : pr.k_off);
-  fft_body<T, POW2>(d, in, out, tw, lb, smem_raw);
+  fft_body<T>(d, in, out, tw, lb, smem_raw);
 }
 
 }  // namespace
 
 int pnh_batch_fft_launch(const BatchProblem* probs, const BatchTable& t, int axis,
-                         int kind, int fp64, int pow2, size_t lds, int threads,
+                         int kind, int fp64, size_t lds, int threads,
                          const void* in, int in_image, void* out, int out_image,
                          const int* done, const int* all_done, hipStream_t s) {
   if (t.n_blocks == 0) return 0;
-  dim3 g((unsigned)t.n_blocks), b(threads);
-  if (fp64) {
-    if (pow2) hipLaunchKernelGGL((fft_batch_kernel<double, true>), g, b, lds, s, probs, t, axis, kind, in, in_image, out, out_image, done, all_done);
-    else hipLaunchKernelGGL((fft_batch_kernel<double, false>), g, b, lds, s, probs, t, axis, kind, in, in_image, out, out_image, done, all_done);
-  } else {
-    if (pow2) hipLaunchKernelGGL((fft_batch_kernel<float, true>), g, b, lds, s, probs, t, axis, kind, in, in_image, out, out_image, done, all_done);
-    else hipLaunchKernelGGL((fft_batch_kernel<float, false>), g, b, lds, s, probs, t, axis, kind, in, in_image, out, out_image, done, all_done);
-  }
-  PNH_LAUNCH_CHECK();
-  return 0;
+  auto go = [&](auto kern) {
+    pnh_fft_allow_lds((const void*)kern, lds);
+    hipLaunchKernelGGL(kern, dim3((unsigned)t.n_blocks), dim3(threads), lds, s, probs, t, axis,
+                       kind, in, in_image, out, out_image, done, all_done);
+    PNH_LAUNCH_CHECK();
+    return 0;
+  };
+  return fp64 ? go(fft_batch_kernel<double>) : go(fft_batch_kernel<float>);
 }
