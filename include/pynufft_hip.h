@@ -130,6 +130,34 @@ typedef struct pnh_plan_desc {
   double row_bound;
 } pnh_plan_desc;
 
+/*
+ * Real factors of a plan (per-axis factors only).  With om the sample's
+ * coordinate, N = Nd[d], K = Kd[d] and b its first support cell,
+ *   u_d[j] = c_d[j] exp(i om / 2) exp(i pi (N - 1) (b + j) / K), c_d[j] real
+ * (b + j not wrapped; the sign (-1)^(N - 1) per wrap of the first cell
+ * belongs to c_d).  The operators then work on a grid modulated by
+ * mod_d[t] = exp(i pi (N - 1) t / K) along every axis, which the FFT passes
+ * read and write, with half the factor bytes and arithmetic.  The stage
+ * entry points (pnh_xx2k, pnh_k2y, pnh_y2k, pnh_k2y2k, pnh_k2xx) keep the
+ * plain grid.  No counterpart in the reference (an implementation choice).
+ *
+ * Records are in row order, 16-byte aligned, x_d = first support cell minus
+ * the tile's origin:
+ *   rec_f32: [M][W] float, W = sum(Jd) + 4 (+ 1 for 3 dims) rounded up to a
+ *     multiple of 4: c_0, c_1, c_2, re and im of exp(i sum_d om_d / 2), then as
+ *     int32 bits x_0 | x_1 << 16, x_2 (3 dims only), the sample index;
+ *   rec_f64: [M][V] double, V = sum(Jd) + 1 rounded up to even: c_0, c_1, c_2,
+ *     then as int64 bits x_0 | x_1 << 16 | x_2 << 32 (NULL: no FP64 operators);
+ *   phase_f64: [M] complex128 exp(i sum_d om_d / 2) (with rec_f64).
+ */
+typedef struct pnh_real_factors {
+  const void* rec_f32;
+  const void* rec_f64;
+  const void* phase_f64;
+  const void* mod_c64[PNH_MAXD];   /* [Kd[d]] complex64 */
+  const void* mod_c128[PNH_MAXD];  /* [Kd[d]] complex128 (with rec_f64) */
+} pnh_real_factors;
+
 typedef struct pnh_plan pnh_plan;
 
 /* Library version string. */
@@ -144,6 +172,12 @@ int pnh_device_count(void);
  * pointers must stay valid for the plan's lifetime.
  * Replaces the offload step of reference nufft/_nufft_class_methods_device.py:183-254. */
 int pnh_plan_create(const pnh_plan_desc* desc, pnh_plan** out);
+/* A plan with real factors.  `desc` may then leave base, u_c64, u_c128 and
+ * csr_c64 NULL (u_c64, base and du_c64 serve pnh_forward_grad_om only); the
+ * complex64 gridding needs item_bound, from pnh_item_bounds on a plan made
+ * without it.  Same checks and reference as pnh_plan_create. */
+int pnh_plan_create_real(const pnh_plan_desc* desc, const pnh_real_factors* real,
+                         pnh_plan** out);
 int pnh_plan_destroy(pnh_plan* plan);
 /* Bytes of `ws` needed by operator `op` in precision `dtype`. */
 int pnh_workspace_bytes(const pnh_plan* plan, int op, int dtype, size_t* bytes);
@@ -322,6 +356,12 @@ typedef struct pnh_graph pnh_graph;
 int pnh_batch_table_bytes(const pnh_plan_desc* descs, int n, size_t* bytes);
 int pnh_batch_create(const pnh_plan_desc* descs, int n, void* table, void* stream,
                      pnh_batch** out);
+/* The same for problems with real factors (real: [n]; complex64 and
+ * complex128, every desc with item_bound). */
+int pnh_batch_table_bytes_real(const pnh_plan_desc* descs, const pnh_real_factors* real, int n,
+                               size_t* bytes);
+int pnh_batch_create_real(const pnh_plan_desc* descs, const pnh_real_factors* real, int n,
+                          void* table, void* stream, pnh_batch** out);
 int pnh_batch_destroy(pnh_batch* batch);
 /* Packed totals: sum of prod(Nd), of M and of prod(Kd). */
 int pnh_batch_sizes(const pnh_batch* batch, int64_t* n_image, int64_t* n_samples,

@@ -59,6 +59,16 @@ class PlanDesc(ctypes.Structure):
     ]
 
 
+class RealFactors(ctypes.Structure):
+    _fields_ = [
+        ('rec_f32', _vp),
+        ('rec_f64', _vp),
+        ('phase_f64', _vp),
+        ('mod_c64', _vp * MAXD),
+        ('mod_c128', _vp * MAXD),
+    ]
+
+
 class HipError(RuntimeError):
     """A HIP runtime failure reported by the library."""
 
@@ -70,6 +80,8 @@ EXPORTS = {
     'pnh_last_error': (ctypes.c_char_p, []),
     'pnh_device_count': (ctypes.c_int, []),
     'pnh_plan_create': (ctypes.c_int, [ctypes.POINTER(PlanDesc), ctypes.POINTER(_vp)]),
+    'pnh_plan_create_real': (ctypes.c_int, [ctypes.POINTER(PlanDesc),
+                                            ctypes.POINTER(RealFactors), ctypes.POINTER(_vp)]),
     'pnh_plan_destroy': (ctypes.c_int, [_vp]),
     'pnh_workspace_bytes': (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int,
                                            ctypes.POINTER(ctypes.c_size_t)]),
@@ -117,6 +129,12 @@ EXPORTS = {
                                              ctypes.POINTER(ctypes.c_size_t)]),
     'pnh_batch_create': (ctypes.c_int, [ctypes.POINTER(PlanDesc), ctypes.c_int, _vp, _vp,
                                         ctypes.POINTER(_vp)]),
+    'pnh_batch_table_bytes_real': (ctypes.c_int, [ctypes.POINTER(PlanDesc),
+                                                  ctypes.POINTER(RealFactors), ctypes.c_int,
+                                                  ctypes.POINTER(ctypes.c_size_t)]),
+    'pnh_batch_create_real': (ctypes.c_int, [ctypes.POINTER(PlanDesc),
+                                             ctypes.POINTER(RealFactors), ctypes.c_int, _vp,
+                                             _vp, ctypes.POINTER(_vp)]),
     'pnh_batch_destroy': (ctypes.c_int, [_vp]),
     'pnh_batch_sizes': (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int64),
                                        ctypes.POINTER(ctypes.c_int64),

@@ -212,7 +212,7 @@ def tune_batch(batch, problems, host_plans, iters=3, reps=2, cache=True, verbose
                     'chunk': hit['chunk'], 'threads': int(hit['threads']),
                     'ms': float(hit['ms'])}
     g = torch.Generator().manual_seed(12345)
-    best = None
+    best = default_ms = None
     import concurrent.futures
     pool = concurrent.futures.ThreadPoolExecutor(8)
     for tile, chunk, thr in batch_candidates(problems):
@@ -226,8 +226,12 @@ def tune_batch(batch, problems, host_plans, iters=3, reps=2, cache=True, verbose
         if verbose:
             print('tune_batch: tile %s chunk %s threads %d -> %.3f ms' % (tile, chunk, thr, ms),
                   flush=True)
-        if best is None or ms < best['ms']:
+        # the first candidate is the defaults: they are left for a clear gain
+        # only (timing noise is a few per cent), as a batch of default work
+        # lists gives the bits of the single problems' solves
+        if best is None or ms < min(best['ms'], 0.92 * default_ms):
             best = {'tile': tile, 'chunk': chunk, 'threads': thr, 'ms': ms}
+            default_ms = best['ms'] if default_ms is None else default_ms
     pool.shutdown()
     batch.release()
     if cache:

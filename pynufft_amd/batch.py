@@ -96,14 +96,23 @@ class BatchNUFFT:
         self.Kd = [op.Kd for op in self.ops]
         self.M = [op.M[0] for op in self.ops]
         self._descs = (_lib.PlanDesc * n)(*[op._desc for op in self.ops])
+        reals = [op._real_desc for op in self.ops]
+        self._reals = None if any(r is None for r in reals) else \
+            (_lib.RealFactors * n)(*reals)
+        if self._reals is None:
+            # one set of kernels for all problems: the complex factors'
+            for i, op in enumerate(self.ops):
+                self._descs[i] = op._complex_desc()
         nbytes = ctypes.c_size_t()
-        _lib.check(self._libh.pnh_batch_table_bytes(self._descs, n, ctypes.byref(nbytes)))
+        _lib.check(self._libh.pnh_batch_table_bytes_real(self._descs, self._reals, n,
+                                                         ctypes.byref(nbytes)))
         self._table = torch.empty(max(256, nbytes.value), dtype=torch.uint8,
                                   device=self.device)
         h = ctypes.c_void_p()
         with torch.cuda.device(self.device):
-            _lib.check(self._libh.pnh_batch_create(self._descs, n, _ptr(self._table),
-                                                   self._stream(), ctypes.byref(h)))
+            _lib.check(self._libh.pnh_batch_create_real(self._descs, self._reals, n,
+                                                        _ptr(self._table), self._stream(),
+                                                        ctypes.byref(h)))
         self._h = h
         ni, ns, ng = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64()
         _lib.check(self._libh.pnh_batch_sizes(h, ctypes.byref(ni), ctypes.byref(ns),

@@ -12,8 +12,11 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB = os.path.join(HERE, 'libpynufft_hip.so')
-# source, object, extra flags; the FFT lengths' kernels in parts (PNH_CT_PARTS)
+# source, object, extra flags; the real-factor kernels by dimension, the FFT
+# lengths' kernels in parts (PNH_CT_PARTS)
 SOURCES = [(s + '.hip', s + '.o', []) for s in ('interp', 'api', 'fft', 'vec', 'solvers')] + \
+    [('real.hip', 'real%dd%d.o' % (d, b), ['-DPNH_D=%d' % d, '-DPNH_F64=%d' % (b == 64)])
+     for d in (3, 2, 1) for b in (64, 32)] + \
     [('fft_ct.hip', 'fft_ct%d.o' % k, ['-DPNH_CT_PART=%d' % k]) for k in range(7)]
 ARCH = os.environ.get('PYNUFFT_HIP_ARCH', 'gfx950')
 

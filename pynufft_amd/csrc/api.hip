@@ -10,6 +10,7 @@
 #include "common.h"
 #include "fft.h"
 #include "interp.h"
+#include "real.h"
 #include "solvers.h"
 #include "vec.h"
 
@@ -46,6 +47,10 @@ struct pnh_plan {
   // [precision][inverse][axis] launch geometry of the FFT passes, made with
   // the plan (n = 0: a length not supported there, refused when it is used)
   FftDesc fft[2][2][PNH_MAXD];
+  // real factors: argument blocks per precision (real[i].rec NULL: none); the
+  // grid inside the operators is then modulated (real.h)
+  RealArgs real[2];
+  const void* mod64[PNH_MAXD];   // complex128 modulation (real factors), or NULL
 };
 
 namespace {
@@ -80,6 +85,7 @@ InterpArgs interp_args(const pnh_plan* p, int fp64) {
 // gridding scratch: item exponents, the row-ordered samples of the exponent
 // pass (long work lists), then the partial slots
 size_t partial_bytes(const pnh_plan* p, int fp64) {
+  if (p->real[fp64].rec) return pnh_real_part_bytes(fp64, p->real[fp64], p->d.n_slots);
   const size_t esz = fp64 ? 16 : 8;
   return pnh_item_exponent_bytes(p->bins.n_items) +
          pnh_row_samples_bytes(p->bins, p->M, p->nb, esz) +
@@ -199,8 +205,10 @@ int build_pass(const pnh_plan* p, int a, bool inverse, bool src_image,
   return 0;
 }
 
+// modulated: the grid is the operators' own (modulated where the plan has real
+// factors of this precision); else the plain spectrum.
 int run_passes_forward(const pnh_plan* p, const void* x_img, void* grid, bool apodize,
-                       int fp64, const int* skip, hipStream_t s) {
+                       int fp64, const int* skip, hipStream_t s, bool modulated) {
   const int D = p->D;
   for (int a = D - 1; a >= 0; --a) {
     FftDesc f;
@@ -208,6 +216,7 @@ int run_passes_forward(const pnh_plan* p, const void* x_img, void* grid, bool ap
     int rc = build_pass(p, a, false, first, false, (first && apodize) ? 1 : 0, fp64,
                         1.0, &f);
     if (rc) return rc;
+    if (modulated && p->real[0].rec) f.mod = fp64 ? p->mod64[a] : p->real[0].mod[a];
     const void* tw = fp64 ? p->d.tw_c128[a] : p->d.tw_c64[a];
     if (!tw) { pnh_set_error("twiddle table missing for axis %d", a); return -1; }
     rc = pnh_fft_launch(f, fp64, first ? x_img : grid, grid, tw, skip, s);
@@ -217,7 +226,7 @@ int run_passes_forward(const pnh_plan* p, const void* x_img, void* grid, bool ap
 }
 
 int run_passes_inverse(const pnh_plan* p, void* grid, void* x_img, bool apodize,
-                       int fp64, const int* skip, hipStream_t s) {
+                       int fp64, const int* skip, hipStream_t s, bool modulated) {
   const int D = p->D;
   for (int a = 0; a < D; ++a) {
     FftDesc f;
@@ -226,6 +235,7 @@ int run_passes_inverse(const pnh_plan* p, void* grid, void* x_img, bool apodize,
     int rc = build_pass(p, a, true, false, last, (last && apodize) ? 2 : 0, fp64,
                         scale, &f);
     if (rc) return rc;
+    if (modulated && p->real[0].rec) f.mod = fp64 ? p->mod64[a] : p->real[0].mod[a];
     const void* tw = fp64 ? p->d.tw_c128[a] : p->d.tw_c64[a];
     if (!tw) { pnh_set_error("twiddle table missing for axis %d", a); return -1; }
     rc = pnh_fft_launch(f, fp64, grid, last ? x_img : grid, tw, skip, s);
@@ -239,6 +249,7 @@ int check_dtype_ready(const pnh_plan* p, int dtype) {
     pnh_set_error("dtype must be PNH_C64 or PNH_C128");
     return -1;
   }
+  if (p->real[dtype == PNH_C128].rec) return 0;
   if (dtype == PNH_C128 && !p->d.u_c128) {
     pnh_set_error("plan has no complex128 factors (u_c128 is NULL)");
     return -1;
@@ -250,41 +261,106 @@ int check_dtype_ready(const pnh_plan* p, int dtype) {
   return 0;
 }
 
+// The operators' gridding and interpolation.  plain: the grid is the caller's
+// plain one (stage entry points); else the operators' own, modulated where
+// the plan has real factors of this precision.
 int do_y2k(const pnh_plan* p, int fp64, const void* y, void* k, void* part,
-           const int* skip, hipStream_t s) {
-  InterpArgs ia = interp_args(p, fp64);
+           const int* skip, hipStream_t s, bool plain = false) {
   if (p->bins.n_items > 0 && !part) {
     pnh_set_error("workspace required for gridding");
     return -1;
   }
+  if (p->real[fp64].rec) {
+    RealArgs a = p->real[fp64];
+    a.stage = plain;
+    REQUIRE(fp64 || a.item_bound || a.n_items == 0,
+            "complex64 gridding with real factors needs item_bound");
+    return pnh_real_y2k(p->D, fp64, a, y, k, part, skip, s);
+  }
+  InterpArgs ia = interp_args(p, fp64);
   return pnh_y2k_launch(ia, p->bins, fp64, y, k, part, skip, s);
 }
 
 int do_k2y(const pnh_plan* p, int fp64, const void* k, void* y, const int* skip,
-           hipStream_t s) {
+           hipStream_t s, bool plain = false) {
+  if (p->real[fp64].rec) {
+    RealArgs a = p->real[fp64];
+    a.stage = plain;
+    return pnh_real_k2y(p->D, fp64, a, k, y, skip, s);
+  }
   InterpArgs ia = interp_args(p, fp64);
   return pnh_k2y_launch(ia, p->bins, fp64, k, y, skip, s);
 }
 
-// k_out = P^H P k, y (samples) receives P k; k_out may alias k
+// k_out = P^H P k, y (samples) is scratch; k_out may alias k
 int do_k2y2k(const pnh_plan* p, int fp64, const void* k, void* y, void* k_out, void* part,
-             const int* skip, hipStream_t s) {
-  InterpArgs ia = interp_args(p, fp64);
+             const int* skip, hipStream_t s, bool plain = false) {
   if (p->bins.n_items > 0 && !part) {
     pnh_set_error("workspace required for gridding");
     return -1;
   }
+  if (p->real[fp64].rec) {
+    RealArgs a = p->real[fp64];
+    a.stage = plain;
+    REQUIRE(fp64 || a.item_bound || a.n_items == 0,
+            "complex64 gridding with real factors needs item_bound");
+    return pnh_real_php(p->D, fp64, a, k, y, k_out, part, skip, s);
+  }
+  InterpArgs ia = interp_args(p, fp64);
   return pnh_k2y2k_launch(ia, p->bins, fp64, k, y, k_out, part, skip, s);
 }
 
+// The argument block of the real factors.
+int real_init(const pnh_plan* p, const pnh_real_factors& r, int fp64, RealArgs* a) {
+  memset(a, 0, sizeof(*a));
+  const void* rec = fp64 ? r.rec_f64 : r.rec_f32;
+  REQUIRE(r.rec_f32 && (r.rec_f64 || !p->d.u_c128),
+          "real factors: rec_f32 is required, and rec_f64 rather than u_c128");
+  if (!rec) return 0;
+  int sj = 0;
+  for (int d = 0; d < p->D; ++d) sj += p->J[d];
+  a->rw = fp64 ? (sj + 2) & ~1 : (sj + 4 + (p->D == 3) + 3) & ~3;
+  for (int d = 0; d < PNH_MAXD; ++d) {
+    const bool on = d < p->D;
+    a->K[d] = on ? (int)p->K[d] : 1;
+    a->J[d] = on ? p->J[d] : 1;
+    a->tile[d] = on ? p->bins.tile[d] : 1;
+    a->tgrid[d] = on ? p->bins.tgrid[d] : 1;
+    a->pad[d] = on ? p->bins.pad[d] : 1;
+    a->flip[d] = on && p->N[d] % 2 == 0;
+    a->mod[d] = on ? (fp64 ? r.mod_c128[d] : r.mod_c64[d]) : nullptr;
+    REQUIRE(!on || a->mod[d], "real factors: mod table of axis %d missing", d);
+    REQUIRE(a->tile[d] < 65536, "real factors: tile of %d cells on axis %d", a->tile[d], d);
+  }
+  REQUIRE(((uintptr_t)rec & 15) == 0, "real factors: records must be 16-byte aligned");
+  REQUIRE(!fp64 || r.phase_f64, "real factors: phase_f64 missing");
+  a->nb = p->nb;
+  a->pad_cells = (int)p->bins.pad_cells;
+  a->max_tile_slots = p->bins.max_tile_slots;
+  a->M = p->M;
+  a->n_items = p->bins.n_items;
+  a->n_tiles = p->bins.n_tiles;
+  a->rec = rec;
+  a->ph = fp64 ? r.phase_f64 : nullptr;
+  a->perm = p->d.perm;
+  a->items = p->bins.items;
+  a->tile_slots = p->bins.tile_slots;
+  a->item_bound = p->bins.item_bound;
+  a->u_bound = p->bins.u_bound;
+  a->row_bound = p->bins.row_bound;
+  a->threads = p->bins.threads;
+  a->k2y_threads = p->bins.k2y_threads;
+  return 0;
+}
 
 // Validate a descriptor and fill a host-side plan (no device work).
-int plan_init(const pnh_plan_desc& d, pnh_plan* p) {
+int plan_init(const pnh_plan_desc& d, pnh_plan* p, const pnh_real_factors* real = nullptr) {
   REQUIRE(d.ndim >= 1 && d.ndim <= PNH_MAXD, "ndim must be 1..%d (got %d)", PNH_MAXD, d.ndim);
   REQUIRE(d.batch >= 1, "batch must be >= 1");
   REQUIRE(d.M >= 0 && d.M < (1LL << 31), "M out of range");
-  REQUIRE(d.perm && d.base, "perm/base pointers are required");
-  REQUIRE(d.u_c64 || d.u_c128 || d.csr_c64, "no interpolator data");
+  REQUIRE(d.perm && (d.base || real), "perm/base pointers are required");
+  REQUIRE(d.u_c64 || d.u_c128 || d.csr_c64 || (real && real->rec_f32), "no interpolator data");
+  REQUIRE(!real || !d.csr_c64, "real factors and a coefficient table exclude each other");
   REQUIRE(!d.csr_c64 || d.csr_col, "csr_col required with csr_c64");
   REQUIRE(d.sn_f32, "sn_f32 is required");
   memset(p, 0, sizeof(*p));
@@ -363,6 +439,12 @@ int plan_init(const pnh_plan_desc& d, pnh_plan* p) {
     p->bins.threads = bytes > 81920 ? 1024 : (bytes > 40960 ? mid : 256);
     const int64_t kbytes = pad_cells * 16;
     p->bins.k2y_threads = kbytes > 81920 ? 1024 : (kbytes > 40960 ? 512 : 256);
+    // several coils multiply an item's rows and its box: 2-D 512x512, 8 coils,
+    // 131 072 samples: k2y 17.6 us at 256 threads, 13.6 at 512, y2k 25.3, 23.7
+    if (real && p->nb >= 4) {
+      p->bins.threads = std::max(p->bins.threads, 512);
+      p->bins.k2y_threads = std::max(p->bins.k2y_threads, 512);
+    }
   } else {
     REQUIRE(d.threads >= 64 && d.threads <= 1024 && d.threads % 64 == 0,
             "threads must be a multiple of 64 in 64..1024 (got %d)", d.threads);
@@ -372,9 +454,15 @@ int plan_init(const pnh_plan_desc& d, pnh_plan* p) {
   p->slot_nbc = p->nb >= 4 ? 4 : (p->nb >= 2 ? 2 : 1);
   REQUIRE(d.fp64_ops == 0 || d.fp64_ops == 1, "fp64_ops must be 0 or 1");
   if (d.fp64_ops) {
-    REQUIRE(d.u_c128 && d.sn_f64, "fp64_ops needs u_c128 and sn_f64");
+    REQUIRE((d.u_c128 || (real && real->rec_f64)) && d.sn_f64, "fp64_ops needs u_c128 and sn_f64");
     for (int a = 0; a < p->D; ++a) REQUIRE(d.tw_c128[a], "fp64_ops needs tw_c128[%d]", a);
   }
+  if (real)
+    for (int fp64 = 0; fp64 < 2; ++fp64) {
+      const int rc = real_init(p, *real, fp64, &p->real[fp64]);
+      if (rc) return rc;
+      for (int a = 0; a < p->D; ++a) p->mod64[a] = real->mod_c128[a];
+    }
   for (int fp64 = 0; fp64 < 2; ++fp64)
     for (int inv = 0; inv < 2; ++inv)
       for (int a = 0; a < p->D; ++a)
@@ -414,7 +502,7 @@ int adjoint_c128(const pnh_plan* p, const void* v, void* x, void* g64, void* img
                  void* part, hipStream_t s) {
   int rc;
   if ((rc = do_y2k(p, 1, v, g64, part, nullptr, s))) return rc;
-  if ((rc = run_passes_inverse(p, g64, img64, false, 1, nullptr, s))) return rc;
+  if ((rc = run_passes_inverse(p, g64, img64, false, 1, nullptr, s, true))) return rc;
   return pnh_cast_mul_sn(img64, x, p->d.sn_f32, p->Ntot, p->nb, s);
 }
 
@@ -429,7 +517,7 @@ int forward_fp64(const pnh_plan* p, const void* x, void* y, void* ws, hipStream_
   void* y64 = w;
   int rc;
   if ((rc = pnh_c64_to_c128(x, x64, p->Ntot * p->nb, s))) return rc;
-  if ((rc = run_passes_forward(p, x64, g64, true, 1, nullptr, s))) return rc;
+  if ((rc = run_passes_forward(p, x64, g64, true, 1, nullptr, s, true))) return rc;
   if (p->M == 0) return 0;
   if ((rc = do_k2y(p, 1, g64, y64, nullptr, s))) return rc;
   return pnh_c128_to_c64(y64, y, p->M * p->nb, s);
@@ -454,9 +542,9 @@ int selfadjoint_fp64(const pnh_plan* p, const void* x, void* x_out, void* ws, hi
   void* part = w;
   int rc;
   if ((rc = pnh_c64_to_c128(x, img64, p->Ntot * p->nb, s))) return rc;
-  if ((rc = run_passes_forward(p, img64, g64, true, 1, nullptr, s))) return rc;
+  if ((rc = run_passes_forward(p, img64, g64, true, 1, nullptr, s, true))) return rc;
   if ((rc = do_k2y2k(p, 1, g64, y64, g64, part, nullptr, s))) return rc;
-  if ((rc = run_passes_inverse(p, g64, img64, false, 1, nullptr, s))) return rc;
+  if ((rc = run_passes_inverse(p, g64, img64, false, 1, nullptr, s, true))) return rc;
   return pnh_cast_mul_sn(img64, x_out, p->d.sn_f32, p->Ntot, p->nb, s);
 }
 
@@ -478,15 +566,20 @@ int pnh_device_count(void) {
   return n;
 }
 
-int pnh_plan_create(const pnh_plan_desc* desc, pnh_plan** out) {
+int pnh_plan_create_real(const pnh_plan_desc* desc, const pnh_real_factors* real,
+                         pnh_plan** out) {
   REQUIRE(desc && out, "null argument");
   *out = nullptr;
   pnh_plan* p = new (std::nothrow) pnh_plan;
   if (!p) { pnh_set_error("out of host memory"); return -1; }
-  const int rc = plan_init(*desc, p);
+  const int rc = plan_init(*desc, p, real);
   if (rc) { delete p; return rc; }
   *out = p;
   return 0;
+}
+
+int pnh_plan_create(const pnh_plan_desc* desc, pnh_plan** out) {
+  return pnh_plan_create_real(desc, nullptr, out);
 }
 
 int pnh_plan_destroy(pnh_plan* plan) {
@@ -494,13 +587,12 @@ int pnh_plan_destroy(pnh_plan* plan) {
   return 0;
 }
 
-// Scratch of density(): ones [M nb], image [N nb], then the adjoint's
-// scratch, which afterwards holds the complex64 grid of the forward FFT.
+// Scratch of density(): samples (complex128), complex64 and complex128 image
+// and grid, gridding partials.
 static size_t density_ws_bytes(const pnh_plan* p) {
-  const size_t adj = adjoint_ws_bytes(p);
-  const size_t grid = align_up((size_t)p->Ktot * p->nb * 8);
-  return align_up((size_t)p->M * p->nb * 8) + align_up((size_t)p->Ntot * p->nb * 8) +
-         (adj > grid ? adj : grid);
+  return align_up((size_t)p->M * p->nb * 16) + align_up((size_t)p->Ntot * p->nb * 8) +
+         align_up((size_t)p->Ntot * p->nb * 16) + align_up((size_t)p->Ktot * p->nb * 8) +
+         align_up((size_t)p->Ktot * p->nb * 16) + align_up(partial_bytes(p, p->d.fp64_ops));
 }
 
 // Scratch of the L1TVOLS solve: uker and |density| (float [K]), images AHy,
@@ -589,6 +681,8 @@ int pnh_workspace_bytes(const pnh_plan* p, int op, int dtype, size_t* bytes) {
 
 int pnh_item_bounds(const pnh_plan* p, double* bound, void* stream) {
   REQUIRE(p && (bound || p->bins.n_items == 0), "null argument");
+  if (p->real[0].rec)
+    return pnh_real_item_bounds(p->D, p->real[0], bound, (hipStream_t)stream);
   REQUIRE(p->d.u_c64, "item bounds need the complex64 factors (u_c64)");
   return pnh_item_bounds_launch(interp_args(p, 0), p->bins, bound, (hipStream_t)stream);
 }
@@ -605,12 +699,12 @@ int pnh_xx2x(const pnh_plan* p, const void* xx, void* x, void* stream) {
 
 int pnh_xx2k(const pnh_plan* p, const void* xx, void* k, void* stream) {
   REQUIRE(p && xx && k, "null argument");
-  return run_passes_forward(p, xx, k, false, 0, nullptr, (hipStream_t)stream);
+  return run_passes_forward(p, xx, k, false, 0, nullptr, (hipStream_t)stream, false);
 }
 
 int pnh_k2xx(const pnh_plan* p, void* k, void* xx, void* stream) {
   REQUIRE(p && xx && k, "null argument");
-  return run_passes_inverse(p, k, xx, false, 0, nullptr, (hipStream_t)stream);
+  return run_passes_inverse(p, k, xx, false, 0, nullptr, (hipStream_t)stream, false);
 }
 
 int pnh_k2y(const pnh_plan* p, int dtype, const void* k, void* y, void* stream) {
@@ -618,14 +712,14 @@ int pnh_k2y(const pnh_plan* p, int dtype, const void* k, void* y, void* stream) 
   int rc = check_dtype_ready(p, dtype);
   if (rc) return rc;
   if (p->M == 0) return 0;
-  return do_k2y(p, dtype == PNH_C128, k, y, nullptr, (hipStream_t)stream);
+  return do_k2y(p, dtype == PNH_C128, k, y, nullptr, (hipStream_t)stream, true);
 }
 
 int pnh_y2k(const pnh_plan* p, int dtype, const void* y, void* k, void* ws, void* stream) {
   REQUIRE(p && k && (y || p->M == 0), "null argument");
   int rc = check_dtype_ready(p, dtype);
   if (rc) return rc;
-  return do_y2k(p, dtype == PNH_C128, y, k, ws, nullptr, (hipStream_t)stream);
+  return do_y2k(p, dtype == PNH_C128, y, k, ws, nullptr, (hipStream_t)stream, true);
 }
 
 int pnh_k2y2k(const pnh_plan* p, int dtype, const void* k, void* k_out, void* ws,
@@ -639,7 +733,7 @@ int pnh_k2y2k(const pnh_plan* p, int dtype, const void* k, void* k_out, void* ws
   void* ytmp = w;
   void* part = w + align_up((size_t)p->M * p->nb * esz);
   hipStream_t s = (hipStream_t)stream;
-  return do_k2y2k(p, fp64, k, ytmp, k_out, part, nullptr, s);
+  return do_k2y2k(p, fp64, k, ytmp, k_out, part, nullptr, s, true);
 }
 
 int pnh_forward(const pnh_plan* p, const void* x, void* y, void* ws, void* stream) {
@@ -648,7 +742,7 @@ int pnh_forward(const pnh_plan* p, const void* x, void* y, void* ws, void* strea
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   if (p->d.fp64_ops) return forward_fp64(p, x, y, ws, s);
-  if ((rc = run_passes_forward(p, x, ws, true, 0, nullptr, s))) return rc;
+  if ((rc = run_passes_forward(p, x, ws, true, 0, nullptr, s, true))) return rc;
   if (p->M == 0) return 0;
   return do_k2y(p, 0, ws, y, nullptr, s);
 }
@@ -663,7 +757,7 @@ int pnh_adjoint(const pnh_plan* p, const void* y, void* x, void* ws, void* strea
   void* grid = w;
   void* part = w + align_up((size_t)p->Ktot * p->nb * 8);
   if ((rc = do_y2k(p, 0, y, grid, part, nullptr, s))) return rc;
-  return run_passes_inverse(p, grid, x, true, 0, nullptr, s);
+  return run_passes_inverse(p, grid, x, true, 0, nullptr, s, true);
 }
 
 int pnh_selfadjoint(const pnh_plan* p, const void* x, void* x_out, void* ws, void* stream) {
@@ -676,9 +770,9 @@ int pnh_selfadjoint(const pnh_plan* p, const void* x, void* x_out, void* ws, voi
   void* grid = w;
   void* ytmp = w + align_up((size_t)p->Ktot * p->nb * 8);
   void* part = (char*)ytmp + align_up((size_t)p->M * p->nb * 8);
-  if ((rc = run_passes_forward(p, x, grid, true, 0, nullptr, s))) return rc;
+  if ((rc = run_passes_forward(p, x, grid, true, 0, nullptr, s, true))) return rc;
   if ((rc = do_k2y2k(p, 0, grid, ytmp, grid, part, nullptr, s))) return rc;
-  return run_passes_inverse(p, grid, x_out, true, 0, nullptr, s);
+  return run_passes_inverse(p, grid, x_out, true, 0, nullptr, s, true);
 }
 
 int pnh_forward_one2many(const pnh_plan* p, const void* x, const void* sense, void* y,
@@ -703,16 +797,45 @@ int pnh_adjoint_many2one(const pnh_plan* p, const void* y, const void* sense, vo
   return pnh_coil_combine(stack, sense, x, p->Ntot, p->nb, (hipStream_t)stream);
 }
 
-// W[i] = |xx2k(adjoint(1))[i]| of the first coil (float [Ktot]).
+// W[i] = |xx2k(adjoint(1))[i]| of the first coil (float [Ktot]).  The FFTs run
+// in FP64, the image between them is rounded to complex64 as the reference's
+// is: the L1-TV solve divides by W - lambda Lap, whose smallest cells multiply
+// an error of W by some 200 (plain 2-D, rho 0.05: 8e-8 in the one cell of
+// W = 0.015 moves the image by 1.3e-5, and the rounding of complex64 FFTs
+// leaves 5e-8 rms in every cell).  Once per solve, some 20 us at a 512x512
+// grid.
 static int density(const pnh_plan* p, float* W, char* w, hipStream_t s) {
-  void* ones = w;
-  void* img = w + align_up((size_t)p->M * p->nb * 8);
-  char* aws = (char*)img + align_up((size_t)p->Ntot * p->nb * 8);   // adjoint scratch, then grid
+  const int64_t my = p->M * p->nb;
+  void* ones = w; w += align_up((size_t)my * 16);
+  void* img = w; w += align_up((size_t)p->Ntot * p->nb * 8);
+  void* img64 = w; w += align_up((size_t)p->Ntot * p->nb * 16);
+  void* g32 = w; w += align_up((size_t)p->Ktot * p->nb * 8);
+  void* g64 = w; w += align_up((size_t)p->Ktot * p->nb * 16);
+  void* part = w;
+  // complex64 FFTs where FP64 has no tables or does not hold the length
+  bool wide = true;
+  for (int a = 0; a < p->D; ++a)
+    wide = wide && p->d.tw_c128[a] && (!p->real[0].rec || p->mod64[a]) && p->fft[1][0][a].n &&
+           p->fft[1][1][a].n;
   int rc;
-  if ((rc = pnh_fill_c64(ones, p->M * p->nb, 1.f, 0.f, s))) return rc;
-  if ((rc = pnh_adjoint(p, ones, img, aws, s))) return rc;
-  if ((rc = run_passes_forward(p, img, aws, false, 0, nullptr, s))) return rc;
-  return pnh_abs_first_coil(aws, W, p->Ktot, p->nb, s);
+  if (p->d.fp64_ops) {
+    if ((rc = pnh_fill_c128(ones, my, 1.0, 0.0, s))) return rc;
+    if ((rc = do_y2k(p, 1, ones, g64, part, nullptr, s))) return rc;
+  } else {
+    if ((rc = pnh_fill_c64(ones, my, 1.f, 0.f, s))) return rc;
+    if ((rc = do_y2k(p, 0, ones, g32, part, nullptr, s))) return rc;
+    if (!wide) {
+      if ((rc = run_passes_inverse(p, g32, img, true, 0, nullptr, s, true))) return rc;
+      if ((rc = run_passes_forward(p, img, g32, false, 0, nullptr, s, false))) return rc;
+      return pnh_abs_first_coil(0, g32, W, p->Ktot, p->nb, s);
+    }
+    if ((rc = pnh_c64_to_c128(g32, g64, p->Ktot * p->nb, s))) return rc;
+  }
+  if ((rc = run_passes_inverse(p, g64, img64, false, 1, nullptr, s, true))) return rc;
+  if ((rc = pnh_cast_mul_sn(img64, img, p->d.sn_f32, p->Ntot, p->nb, s))) return rc;
+  if ((rc = pnh_c64_to_c128(img, img64, p->Ntot * p->nb, s))) return rc;
+  if ((rc = run_passes_forward(p, img64, g64, false, 1, nullptr, s, false))) return rc;
+  return pnh_abs_first_coil(1, g64, W, p->Ktot, p->nb, s);
 }
 
 int pnh_precompute_sp(const pnh_plan* p, float* W, void* ws, void* stream) {
@@ -727,9 +850,9 @@ int pnh_selfadjoint2(const pnh_plan* p, const void* x, const float* W, void* x_o
   REQUIRE(p && x && W && x_out && ws, "null argument");
   hipStream_t s = (hipStream_t)stream;
   int rc;
-  if ((rc = run_passes_forward(p, x, ws, false, 0, nullptr, s))) return rc;
+  if ((rc = run_passes_forward(p, x, ws, false, 0, nullptr, s, false))) return rc;
   if ((rc = pnh_scale_sn(0, ws, ws, W, p->Ktot, p->nb, s))) return rc;
-  return run_passes_inverse(p, ws, x_out, false, 0, nullptr, s);
+  return run_passes_inverse(p, ws, x_out, false, 0, nullptr, s, false);
 }
 
 int pnh_solve_dc(const pnh_plan* p, const void* y, void* x, int maxiter, void* ws,
@@ -754,7 +877,7 @@ int pnh_solve_dc(const pnh_plan* p, const void* y, void* x, int maxiter, void* w
   if ((rc = pnh_fill_c128(W, my, 1.0, 0.0, s))) return rc;
   for (int it = 0; it < maxiter; ++it) {
     if ((rc = adjoint_c128(p, W, x, g64, img64, part, s))) return rc;
-    if ((rc = run_passes_forward(p, x, g32, true, 0, nullptr, s))) return rc;
+    if ((rc = run_passes_forward(p, x, g32, true, 0, nullptr, s, true))) return rc;
     if ((rc = pnh_c64_to_c128(g32, g64, p->Ktot * p->nb, s))) return rc;
     if (p->M > 0 && (rc = do_k2y(p, 1, g64, E, nullptr, s))) return rc;
     if ((rc = pnh_cdiv_c128(W, E, my, s))) return rc;
@@ -803,9 +926,9 @@ int pnh_solve_l1tvols(const pnh_plan* p, const void* y, void* x, int maxiter, do
   const float thr = (float)(1.0 / (double)lam);
   for (int it = 0; it < maxiter; ++it) {
     if ((rc = pnh_l1tv_rhs(AHyk, dd, bb, rhs, gn, mu, lam, s))) return rc;
-    if ((rc = run_passes_forward(p, rhs, sws, false, 0, nullptr, s))) return rc;
+    if ((rc = run_passes_forward(p, rhs, sws, false, 0, nullptr, s, false))) return rc;
     if ((rc = pnh_l1tv_kdiv(sws, uker, K, s))) return rc;
-    if ((rc = run_passes_inverse(p, sws, x, false, 0, nullptr, s))) return rc;
+    if ((rc = run_passes_inverse(p, sws, x, false, 0, nullptr, s, false))) return rc;
     if ((rc = pnh_selfadjoint(p, x, q, sws, s))) return rc;
     if ((rc = pnh_l1tv_shrink(x, q, AHy, AHyk, dd, bb, gn, thr, s))) return rc;
   }
@@ -867,7 +990,7 @@ int pnh_solve_lsqr(const pnh_plan* p, const void* y, void* x, int iter_lim, doub
       if (flag) break;
     }
   }
-  if ((rc = run_passes_inverse(p, xk, img64, false, 1, nullptr, s))) return rc;
+  if ((rc = run_passes_inverse(p, xk, img64, false, 1, nullptr, s, true))) return rc;
   if ((rc = pnh_cast_div_sn(img64, x, p->d.sn_f32, p->Ntot, 1, s))) return rc;
   if (info_out) {
     PNH_CHECK_HIP(hipMemcpyAsync(info_out, &st->istop, sizeof(int), hipMemcpyDeviceToDevice, s));
@@ -930,7 +1053,7 @@ int pnh_solve_lsmr(const pnh_plan* p, const void* y, void* x, int maxiter, doubl
       if (flag) break;
     }
   }
-  if ((rc = run_passes_inverse(p, xk, img64, false, 1, nullptr, s))) return rc;
+  if ((rc = run_passes_inverse(p, xk, img64, false, 1, nullptr, s, true))) return rc;
   if ((rc = pnh_cast_div_sn(img64, x, p->d.sn_f32, p->Ntot, 1, s))) return rc;
   if (info_out) {
     PNH_CHECK_HIP(hipMemcpyAsync(info_out, &st->istop, sizeof(int), hipMemcpyDeviceToDevice, s));
@@ -1005,7 +1128,7 @@ int pnh_solve_bicg(const pnh_plan* p, int kind, const void* y, void* x, int maxi
       if (flag) break;
     }
   }
-  if ((rc = run_passes_inverse(p, xk, img64, false, 1, nullptr, s))) return rc;
+  if ((rc = run_passes_inverse(p, xk, img64, false, 1, nullptr, s, true))) return rc;
   if ((rc = pnh_cast_div_sn(img64, x, p->d.sn_f32, p->Ntot, 1, s))) return rc;
   if (info_out) {
     PNH_CHECK_HIP(hipMemcpyAsync(info_out, &st->info, sizeof(int), hipMemcpyDeviceToDevice, s));
@@ -1098,7 +1221,7 @@ int pnh_solve_gmres(const pnh_plan* p, const void* y, void* x, int restart, int 
       if (flag) break;
     }
   }
-  if ((rc = run_passes_inverse(p, xk, img64, false, 1, nullptr, s))) return rc;
+  if ((rc = run_passes_inverse(p, xk, img64, false, 1, nullptr, s, true))) return rc;
   if ((rc = pnh_cast_div_sn(img64, x, p->d.sn_f32, p->Ntot, 1, s))) return rc;
   if (info_out) {
     PNH_CHECK_HIP(hipMemcpyAsync(info_out, &st->info, sizeof(int), hipMemcpyDeviceToDevice, s));
@@ -1219,7 +1342,7 @@ int pnh_solve_lgmres(const pnh_plan* p, const void* y, void* x, int maxiter, int
       if (flag) break;
     }
   }
-  if ((rc = run_passes_inverse(p, xk, img64, false, 1, nullptr, s))) return rc;
+  if ((rc = run_passes_inverse(p, xk, img64, false, 1, nullptr, s, true))) return rc;
   if ((rc = pnh_cast_div_sn(img64, x, p->d.sn_f32, p->Ntot, 1, s))) return rc;
   if (info_out) {
     PNH_CHECK_HIP(hipMemcpyAsync(info_out, &st->info, sizeof(int), hipMemcpyDeviceToDevice, s));
@@ -1232,7 +1355,7 @@ int pnh_solve_lgmres(const pnh_plan* p, const void* y, void* x, int maxiter, int
 int pnh_forward_grad_om(const pnh_plan* p, const void* k, const void* g, float* om_grad,
                         void* stream) {
   REQUIRE(p && k && (g || p->M == 0) && (om_grad || p->M == 0), "null argument");
-  REQUIRE(p->d.du_c64 && p->d.u_c64, "plan has no factor derivatives (du_c64)");
+  REQUIRE(p->d.du_c64 && p->d.u_c64 && p->d.base, "plan has no factor derivatives (du_c64)");
   InterpArgs ia = interp_args(p, 0);
   return pnh_k2y_dom_launch(ia, 0, k, g, om_grad, (hipStream_t)stream);
 }
@@ -1245,7 +1368,7 @@ static int cg_solve(const pnh_plan* p, const void* y, void* x, int maxiter, doub
   REQUIRE(p && x && ws && (y || p->M == 0), "null argument");
   REQUIRE(maxiter >= 0, "maxiter must be >= 0");
   REQUIRE(p->nb <= PNH_CG_MAXNB, "solve supports at most %d coils", PNH_CG_MAXNB);
-  REQUIRE(p->d.u_c128 && p->d.tw_c128[0] && p->d.sn_f32,
+  REQUIRE((p->d.u_c128 || p->real[1].rec) && p->d.tw_c128[0] && p->d.sn_f32,
           "FP64 solve needs u_c128 and tw_c128 in the plan");
   for (int a = 0; a < p->D; ++a)
     REQUIRE(p->d.tw_c128[a], "tw_c128[%d] missing", a);
@@ -1269,17 +1392,41 @@ static int cg_solve(const pnh_plan* p, const void* y, void* x, int maxiter, doub
   const int64_t K = p->Ktot;
   // b = P^H y in FP64 (y is complex64; upcast exactly as scipy does)
   if (p->M > 0 && (rc = pnh_c64_to_c128(y, yt, p->M * nb, s))) return rc;
-  if ((rc = do_y2k(p, 1, yt, vr, part, nullptr, s))) return rc;
-  if ((rc = pnh_zero(1, vx, K * nb, s))) return rc;
-  if ((rc = pnh_cg_dot(1, vr, vr, K, nb, redp, nullptr, s))) return rc;
-  if ((rc = pnh_cg_init(redp, nb, sc, maxiter, rtol, atol, s))) return rc;
+  // Where the gather can make the steps itself, vq holds its partial sums
+  // (the items' |P p|^2, the workgroups' |r|^2).  512x512, 205 824 samples:
+  // 10 iterations 493 us, with q stored and two more kernels 511.
+  const int64_t blocks = pnh_real_cg_blocks(p->D, p->real[1]);
+  const int64_t n_items = blocks ? p->real[1].n_items : 0;
+  RealCg cg = {};
+  const bool fused = blocks > 0 && (size_t)(n_items + blocks) * 16 <= g2;
+  if (fused) {
+    cg.x = vx;
+    cg.r = vr;
+    cg.p = vp;
+    cg.pq = vq;
+    cg.n_pq = (int)n_items;
+    cg.rr = (char*)vq + n_items * 16;
+    if ((rc = pnh_real_y2k_cg(p->D, p->real[1], yt, part, cg, s))) return rc;
+  } else {
+    if ((rc = do_y2k(p, 1, yt, vr, part, nullptr, s))) return rc;
+    if ((rc = pnh_zero(1, vx, K * nb, s))) return rc;
+    if ((rc = pnh_cg_dot(1, vr, vr, K, nb, redp, nullptr, s))) return rc;
+  }
+  const void* rr = fused ? cg.rr : redp;
+  const int rr_blocks = fused ? (int)blocks : PNH_RED_BLOCKS;
+  if ((rc = pnh_cg_init(rr, rr_blocks, nb, sc, maxiter, rtol, atol, s))) return rc;
   for (int it = 0; it < maxiter; ++it) {
     // the p update finishes the previous iteration's |r|^2 and stopping test
     const int* all_done = &sc->all_done[it & 1];
-    if ((rc = pnh_cg_p_update(vp, vr, K, nb, sc, redp, it, s))) return rc;
-    if ((rc = do_k2y2k(p, 1, vp, yt, vq, part, all_done, s))) return rc;
-    if ((rc = pnh_cg_dot(0, vp, vq, K, nb, redpq, all_done, s))) return rc;
-    if ((rc = pnh_cg_xr_update(vx, vr, vp, vq, K, nb, sc, it, redpq, redp, s))) return rc;
+    if ((rc = pnh_cg_p_update(vp, vr, K, nb, sc, rr, rr_blocks, it, s))) return rc;
+    if (fused) {
+      cg.rho = &sc->rr[it & 1][0];
+      if ((rc = pnh_real_php_cg(p->D, p->real[1], part, cg, all_done, s))) return rc;
+    } else {
+      if ((rc = do_k2y2k(p, 1, vp, yt, vq, part, all_done, s))) return rc;
+      if ((rc = pnh_cg_dot(0, vp, vq, K, nb, redpq, all_done, s))) return rc;
+      if ((rc = pnh_cg_xr_update(vx, vr, vp, vq, K, nb, sc, it, redpq, redp, s))) return rc;
+    }
     if (host_checks && (it & 63) == 63 && it + 1 < maxiter) {
       // long runs: stop launching once every coil has converged (as seen by
       // this iteration's p update)
@@ -1289,14 +1436,15 @@ static int cg_solve(const pnh_plan* p, const void* y, void* x, int maxiter, doub
       if (flag) break;
     }
   }
+  // before the inverse passes use vq
+  if (resid_out && (rc = pnh_cg_resid(rr, rr_blocks, nb, sc, resid_out, s))) return rc;
   // x = complex64(crop(ifftn(k))) / sn, inverse FFT in FP64 (as numpy does
   // for the complex128 CG result)
-  if ((rc = run_passes_inverse(p, vx, vq, false, 1, nullptr, s))) return rc;
+  if ((rc = run_passes_inverse(p, vx, vq, false, 1, nullptr, s, true))) return rc;
   if ((rc = pnh_cast_div_sn(vq, x, p->d.sn_f32, p->Ntot, nb, s))) return rc;
   if (iters_out)
     PNH_CHECK_HIP(hipMemcpyAsync(iters_out, sc->iters, sizeof(int) * nb,
                                  hipMemcpyDeviceToDevice, s));
-  if (resid_out && (rc = pnh_cg_resid(redp, nb, sc, resid_out, s))) return rc;
   return 0;
 }
 
@@ -1377,6 +1525,10 @@ struct pnh_batch {
   int packed;                          // every problem has per-item bounds
   int fixed_pad;                       // every problem's boxes have extent PNH_FIXED_PAD
                                        // and every problem a row bound
+  int real;                            // every problem has real factors
+  int cg_steps;                        // the gather makes the steps of the solve
+  int layout;                          // how their supports lie in the boxes (batch.h)
+  int row_bounds;                      // every problem has a row bound
   int J[PNH_MAXD];
   int64_t N_total, M_total, K_total, part_elems, pad_cells_max;
   int fft_threads;
@@ -1397,7 +1549,7 @@ struct pnh_graph {
 
 namespace {
 
-const int64_t kVecChunk = 4096;
+const int64_t kVecChunk = 1024;
 
 struct Blob {
   std::vector<unsigned char> bytes;
@@ -1427,17 +1579,19 @@ void add_table(Blob& blob, const std::vector<int64_t>& blocks_per_problem,
 
 // Build every host-side table of a batch.  With `table` NULL only sizes are
 // computed; otherwise the blob is copied to `table` and device pointers set.
-int build_batch(const pnh_plan_desc* descs, int n, void* table, hipStream_t stream,
-                pnh_batch* b) {
+int build_batch(const pnh_plan_desc* descs, const pnh_real_factors* real, int n, void* table,
+                hipStream_t stream, pnh_batch* b) {
   REQUIRE(descs && n >= 1, "need at least one problem");
   memset(b, 0, sizeof(*b));
   std::vector<pnh_plan> plans(n);
   for (int i = 0; i < n; ++i) {
-    int rc = plan_init(descs[i], &plans[i]);
+    int rc = plan_init(descs[i], &plans[i], real ? real + i : nullptr);
     if (rc) return rc;
     const pnh_plan& p = plans[i];
     REQUIRE(p.nb == 1, "batched problems are single-coil (problem %d has batch %d)", i, p.nb);
-    REQUIRE(p.d.u_c64 && p.d.u_c128 && p.d.tw_c128[0], "problem %d lacks c64/c128 factors", i);
+    REQUIRE((real ? p.real[0].rec && p.real[1].rec : p.d.u_c64 && p.d.u_c128) && p.d.tw_c128[0],
+            "problem %d lacks c64/c128 factors", i);
+    REQUIRE(!real || p.bins.item_bound || p.bins.n_items == 0, "problem %d lacks item_bound", i);
     REQUIRE(!p.d.csr_c64, "batched problems use the per-axis factors");
     REQUIRE(!p.d.fp64_ops, "problem %d needs FP64 operators (fp64_ops); batches run the "
             "complex64 operators in FP32", i);
@@ -1465,10 +1619,20 @@ int build_batch(const pnh_plan_desc* descs, int n, void* table, hipStream_t stre
     if (!plans[i].bins.item_bound && plans[i].bins.n_items > 0) b->packed = 0;
     if (!pnh_fixed_pad(plans[i].bins, D) || !(plans[i].bins.row_bound > 0.0)) b->fixed_pad = 0;
   }
+  b->real = real != nullptr;
+  b->layout = D >= 2 ? 1 : -1;
+  b->row_bounds = 1;
+  for (int i = 0; i < n; ++i) {
+    b->row_bounds &= plans[i].bins.row_bound > 0.0;
+    for (int a = 0; a < D; ++a) {
+      if (plans[i].bins.tgrid[a] == 1) b->layout = 0;
+      if (b->layout > 0 && plans[i].bins.pad[a] != 15 + plans[i].J[a]) b->layout = -1;
+    }
+  }
   b->fft_threads = 256;
   b->vec_chunk = kVecChunk;
   std::vector<BatchProblem> probs(n);
-  int64_t xo = 0, yo = 0, ko = 0, so = 0;
+  int64_t xo = 0, yo = 0, ko = 0, so = 0, io = 0;
   for (int i = 0; i < n; ++i) {
     const pnh_plan& p = plans[i];
     BatchProblem& q = probs[i];
@@ -1476,7 +1640,10 @@ int build_batch(const pnh_plan_desc* descs, int n, void* table, hipStream_t stre
     q.ia = interp_args(&p, 0);
     q.ia64 = interp_args(&p, 1);
     q.bins = p.bins;
-    q.x_off = xo; q.y_off = yo; q.k_off = ko; q.part_off = so;
+    q.ra = p.real[0];
+    q.ra64 = p.real[1];
+    q.ra.cl = q.ra64.cl = 1;
+    q.x_off = xo; q.y_off = yo; q.k_off = ko; q.part_off = so; q.item_off = io;
     q.n_img = p.Ntot;
     q.n_grid = p.Ktot;
     q.sn32 = p.d.sn_f32;
@@ -1488,21 +1655,32 @@ int build_batch(const pnh_plan_desc* descs, int n, void* table, hipStream_t stre
                                false);
       if (!rc) rc = build_pass(&p, a, true, false, a == D - 1, 0, 1, sc, &q.inv64[a], false);
       if (rc) return rc;
+      q.fwd[a].mod = q.inv[a].mod = p.real[0].mod[a];     // null without real factors
+      q.inv64[a].mod = p.real[1].mod[a];
       q.tw32[a] = p.d.tw_c64[a];
       q.tw64[a] = p.d.tw_c128[a];
     }
     xo += p.Ntot; yo += p.M; ko += p.Ktot; so += p.d.n_slots * p.bins.pad_cells;
+    io += p.d.n_items;
   }
   b->N_total = xo; b->M_total = yo; b->K_total = ko; b->part_elems = so;
 
   Blob blob;
   const size_t off_probs = blob.add(probs.data(), probs.size() * sizeof(BatchProblem));
-  // gridding gather: pnh_gather_parts blocks per tile
+  // gridding gather: blocks per tile
   std::vector<int64_t> nb_tiles(n);
   for (int i = 0; i < n; ++i)
-    nb_tiles[i] = plans[i].bins.n_tiles * pnh_gather_parts(plans[i].bins);
+    nb_tiles[i] = plans[i].bins.n_tiles * (real ? pnh_real_gather_parts(probs[i].ra, D)
+                                                : pnh_gather_parts(plans[i].bins));
   size_t og_tab, og_first;
   add_table(blob, nb_tiles, &og_tab, &og_first, &b->gather_t.n_blocks);
+  // every problem's conjugate gradients can take pnh_real_cg_blocks' steps,
+  // and their partial sums fit where q would be (a problem without samples
+  // has a zero right side and no steps)
+  b->cg_steps = real && b->row_bounds && io + b->gather_t.n_blocks <= ko;
+  for (int i = 0; i < n; ++i)
+    if (plans[i].d.n_items > 0 && pnh_real_cg_blocks(D, probs[i].ra64) == 0) b->cg_steps = 0;
+  if ((size_t)b->pad_cells_max * 32 + 256 > pnh_lds_limit()) b->cg_steps = 0;
   // FFT passes per kind and axis
   size_t of_tab[3][PNH_MAXD], of_first[3][PNH_MAXD];
   for (int kind = 0; kind < 3; ++kind)
@@ -1594,7 +1772,11 @@ int batch_passes(const pnh_batch* b, int kind, int fp64, const void* image_in,
 }
 
 int batch_y2k(const pnh_batch* b, int fp64, const void* y, void* k, void* part,
-              const int* done, const int* all_done, hipStream_t s) {
+              const int* done, const int* all_done, const RealBatchCg* cg, hipStream_t s) {
+  if (b->real)
+    return pnh_real_batch_y2k(b->D, fp64, b->J, b->layout, b->probs, b->items, b->n_items,
+                              b->gather_t, b->pad_cells_max, b->grid_threads, y, k, part, done,
+                              all_done, cg, s);
   return pnh_batch_y2k_launch(b->probs, b->items, b->n_items, b->gather_t,
                               b->D, b->J, fp64, b->packed, b->pad_cells_max, b->grid_threads,
                               y, k, part, done, all_done, s);
@@ -1647,52 +1829,87 @@ int batch_solve(const pnh_batch* b, const void* y, void* x, int maxiter, double 
   // b = P^H y in FP64 (complex64 samples upcast exactly) into r, x = 0, |b|^2
   if ((rc = pnh_batch_vec_launch(BVEC_CAST_Y, b->probs, b->vec_t[1], ch, (void*)y, w.yt,
                                  nullptr, nullptr, cg, 0, s))) return rc;
-  if ((rc = batch_y2k(b, 1, w.yt, w.r, w.part, nullptr, nullptr, s))) return rc;
-  if ((rc = pnh_batch_vec_launch(BVEC_ZERO_X, b->probs, gt, ch, w.x, nullptr, nullptr,
-                                 nullptr, cg, 0, s))) return rc;
-  if ((rc = pnh_batch_vec_launch(BVEC_DOT_RR, b->probs, gt, ch, w.r, nullptr, nullptr,
-                                 nullptr, cg, 0, s))) return rc;
+  // (cg_steps: the gather makes the steps, as cg_solve's)
+  RealBatchCg rc_ = {};
+  const RealBatchCg* steps = nullptr;
+  if (b->cg_steps) {
+    rc_.x = (double2*)w.x;
+    rc_.r = (double2*)w.r;
+    rc_.p = (const double2*)w.p;
+    rc_.pq = (double2*)w.q;
+    rc_.rr = rc_.pq + b->n_items;
+    cg.part_rr = rc_.rr;
+    cg.rr_t = b->gather_t;
+    steps = &rc_;
+  } else {
+    cg.rr_t = gt;
+  }
+  if ((rc = batch_y2k(b, 1, w.yt, w.r, w.part, nullptr, nullptr, steps, s))) return rc;
+  if (!steps) {
+    if ((rc = pnh_batch_vec_launch(BVEC_ZERO_X, b->probs, gt, ch, w.x, nullptr, nullptr,
+                                   nullptr, cg, 0, s))) return rc;
+    if ((rc = pnh_batch_vec_launch(BVEC_DOT_RR, b->probs, gt, ch, w.r, nullptr, nullptr,
+                                   nullptr, cg, 0, s))) return rc;
+  }
   for (int it = 0; it < maxiter; ++it) {
     // the p update finishes the previous iteration's |r|^2 and stopping test
     const int* done = cg.done + (it & 1) * b->n;
+    rc_.rho = cg.rr + (it & 1) * b->n;
     if ((rc = pnh_batch_vec_launch(BVEC_P_UPDATE, b->probs, gt, ch, w.p, w.r, nullptr,
                                    nullptr, cg, it, s))) return rc;
-    if ((rc = pnh_batch_k2y2k_launch(b->probs, b->items, b->n_items, b->gather_t, b->D, b->J,
-                                     1, b->pad_cells_max, b->grid_threads, b->fixed_pad, w.p,
-                                     w.yt, w.q, w.part, done, nullptr, s))) return rc;
+    rc = b->real ? pnh_real_batch_php(b->D, b->J, b->layout, b->row_bounds, b->probs, b->items,
+                                      b->n_items, b->gather_t, b->pad_cells_max,
+                                      b->grid_threads, w.p, w.yt, w.q, w.part, done, nullptr,
+                                      steps, s)
+                 : pnh_batch_k2y2k_launch(b->probs, b->items, b->n_items, b->gather_t, b->D, b->J,
+                                          1, b->pad_cells_max, b->grid_threads, b->fixed_pad,
+                                          w.p, w.yt, w.q, w.part, done, nullptr, s);
+    if (rc) return rc;
+    if (steps) continue;
     if ((rc = pnh_batch_vec_launch(BVEC_DOT_PQ, b->probs, gt, ch, w.p, w.q, nullptr,
                                    nullptr, cg, it, s))) return rc;
     if ((rc = pnh_batch_vec_launch(BVEC_XR_UPDATE, b->probs, gt, ch, w.x, w.r, w.p,
                                    w.q, cg, it, s))) return rc;
   }
+  // before the inverse passes use q
+  if ((rc = pnh_batch_cg_out_launch(cg, iters_out, resid_out, s))) return rc;
   // image = crop(ifftn(k)) in FP64 into q (packed image layout), then
   // x = complex64(image) / sn
   if ((rc = batch_passes(b, BFFT_INV64, 1, nullptr, w.q, w.x, nullptr, nullptr, s))) return rc;
-  if ((rc = pnh_batch_vec_launch(BVEC_CAST_DIV, b->probs, b->vec_t[2], ch, w.q, x, nullptr,
-                                 nullptr, cg, 0, s))) return rc;
-  return pnh_batch_cg_out_launch(gt, cg, iters_out, resid_out, s);
+  return pnh_batch_vec_launch(BVEC_CAST_DIV, b->probs, b->vec_t[2], ch, w.q, x, nullptr, nullptr,
+                              cg, 0, s);
 }
 
 }  // namespace
 
 extern "C" {
 
-int pnh_batch_table_bytes(const pnh_plan_desc* descs, int n, size_t* bytes) {
+int pnh_batch_table_bytes_real(const pnh_plan_desc* descs, const pnh_real_factors* real, int n,
+                               size_t* bytes) {
   REQUIRE(bytes, "null argument");
   pnh_batch b;
-  int rc = build_batch(descs, n, nullptr, nullptr, &b);
+  int rc = build_batch(descs, real, n, nullptr, nullptr, &b);
   if (rc) return rc;
   *bytes = b.table_bytes;
   return 0;
 }
 
+int pnh_batch_table_bytes(const pnh_plan_desc* descs, int n, size_t* bytes) {
+  return pnh_batch_table_bytes_real(descs, nullptr, n, bytes);
+}
+
 int pnh_batch_create(const pnh_plan_desc* descs, int n, void* table, void* stream,
                      pnh_batch** out) {
+  return pnh_batch_create_real(descs, nullptr, n, table, stream, out);
+}
+
+int pnh_batch_create_real(const pnh_plan_desc* descs, const pnh_real_factors* real, int n,
+                          void* table, void* stream, pnh_batch** out) {
   REQUIRE(out && table, "null argument");
   *out = nullptr;
   pnh_batch* b = new (std::nothrow) pnh_batch;
   if (!b) { pnh_set_error("out of host memory"); return -1; }
-  int rc = build_batch(descs, n, table, (hipStream_t)stream, b);
+  int rc = build_batch(descs, real, n, table, (hipStream_t)stream, b);
   if (rc) { delete b; return rc; }
   *out = b;
   return 0;
@@ -1730,6 +1947,9 @@ int pnh_batch_forward(const pnh_batch* b, const void* x, void* y, void* ws, void
   hipStream_t s = (hipStream_t)stream;
   int rc = batch_passes(b, BFFT_FWD, 0, x, nullptr, ws, nullptr, nullptr, s);
   if (rc) return rc;
+  if (b->real)
+    return pnh_real_batch_k2y(b->D, b->J, b->layout, b->probs, b->items, b->n_items,
+                              b->pad_cells_max, b->grid_threads, ws, y, nullptr, nullptr, s);
   return pnh_batch_k2y_launch(b->probs, b->items, b->n_items, b->D, b->J, 0,
                               b->pad_cells_max, b->grid_threads, ws, y, nullptr, nullptr, s);
 }
@@ -1740,7 +1960,7 @@ int pnh_batch_adjoint(const pnh_batch* b, const void* y, void* x, void* ws, void
   char* w = (char*)ws;
   void* grid = w;
   void* part = w + align_up((size_t)b->K_total * 8);
-  int rc = batch_y2k(b, 0, y, grid, part, nullptr, nullptr, s);
+  int rc = batch_y2k(b, 0, y, grid, part, nullptr, nullptr, nullptr, s);
   if (rc) return rc;
   return batch_passes(b, BFFT_INV, 0, nullptr, x, grid, nullptr, nullptr, s);
 }

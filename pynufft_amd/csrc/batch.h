@@ -3,6 +3,7 @@
 #include "common.h"
 #include "fft.h"
 #include "interp.h"
+#include "real.h"
 
 // One problem of a batch, resident in device memory.  Vector offsets are in
 // complex elements of the packed batch vectors (problems back to back).
@@ -10,8 +11,10 @@ struct BatchProblem {
   InterpArgs ia;             // complex64 factors
   InterpArgs ia64;           // complex128 factors
   BinArgs bins;              // this problem's gridding work list
+  RealArgs ra, ra64;         // real factors (rec NULL: none), one coil
   int64_t x_off, y_off, k_off;
   int64_t part_off;          // first element of this problem's partial slots
+  int64_t item_off;          // items of the problems before this one
   int64_t n_img, n_grid;     // prod(Nd), prod(Kd)
   const float* sn32;
   FftDesc fwd[PNH_MAXD];     // forward passes, fp32, x2xx fused in the first
@@ -45,6 +48,7 @@ struct BatchCg {
   double* res;
   double2* part_rr;          // |r|^2 (|b|^2 before the first iteration)
   double2* part_pq;          // p . q
+  BatchTable rr_t;           // blocks of part_rr
   int n;
   int maxiter;
   double rtol, atol;
@@ -81,8 +85,38 @@ int pnh_batch_vec_launch(int op, const BatchProblem* probs, const BatchTable& t,
                          const BatchCg& cg, int it, hipStream_t s);
 // Iterations run and final ||r|| per problem (either output may be null);
 // t is the grid table whose block partials the last CG step wrote.
-int pnh_batch_cg_out_launch(const BatchTable& t, const BatchCg& cg, int32_t* iters_out,
+int pnh_batch_cg_out_launch(const BatchCg& cg, int32_t* iters_out,
                             double* resid_out, hipStream_t s);
+
+// The gridding as a step of the conjugate gradients (RealCg), packed vectors:
+// pq per item (item_off + item), rr per block of the gather table, rho per
+// problem.
+struct RealBatchCg {
+  double2 *x, *r;
+  const double2* p;
+  double2* pq;
+  const double* rho;
+  double2* rr;
+};
+
+// The same with real factors, on modulated grids (real.hip).  layout: how
+// the supports lie in every problem's boxes (real.hip, layout_of).
+int pnh_real_batch_k2y(int D, const int* J, int layout, const BatchProblem* probs,
+                       const int2* items, int64_t n_items, int64_t pad_cells, int threads,
+                       const void* k, void* y, const int* done, const int* all_done,
+                       hipStream_t s);
+int pnh_real_batch_y2k(int D, int fp64, const int* J, int layout, const BatchProblem* probs,
+                       const int2* items, int64_t n_items, const BatchTable& gather,
+                       int64_t pad_cells, int threads, const void* y, void* k, void* part,
+                       const int* done, const int* all_done, const RealBatchCg* cg,
+                       hipStream_t s);
+// bounds: every problem has a row bound.  cg (or null): the gather makes a
+// step of the conjugate gradients in place of k_out.
+int pnh_real_batch_php(int D, const int* J, int layout, int bounds, const BatchProblem* probs,
+                       const int2* items, int64_t n_items, const BatchTable& gather,
+                       int64_t pad_cells, int threads, const void* k, void* ybuf, void* k_out,
+                       void* part, const int* done, const int* all_done, const RealBatchCg* cg,
+                       hipStream_t s);
 
 enum { BFFT_FWD = 0, BFFT_INV = 1, BFFT_INV64 = 2 };
 enum { BVEC_CAST_Y = 0, BVEC_ZERO_X = 1, BVEC_DOT_RR = 2, BVEC_P_UPDATE = 3,

@@ -34,6 +34,10 @@ struct FftDesc {
   const void* sn;       // real apodization (float or double, matches dtype)
   int64_t sn_o_stride[2];
   int64_t sn_t_stride;
+  // per-point factor along the transformed axis (complex, matches dtype), or
+  // NULL: the forward transform multiplies point t of its output by mod[t],
+  // the inverse point t of its input by conj(mod[t])
+  const void* mod;
   int npass;
   uint64_t radices;     // pass p's radix - 1 in bits 4p .. 4p + 3
   int lines_per_block;

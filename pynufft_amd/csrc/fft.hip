@@ -132,6 +132,11 @@ __device__ __forceinline__ void fft_body(const FftDesc& d, const void* in_, void
         const T s = ((const T*)d.sn)[li.sn + (int64_t)t * d.sn_t_stride];
         v.x *= s; v.y *= s;
       }
+      if (d.mod && d.sign > 0) {
+        C m = ((const C*)d.mod)[t];
+        m.y = -m.y;
+        v = cmul_fma(v, m);
+      }
     }
     v.y *= cj;
     src[l * ld + t + (t >> 4)] = v;
@@ -166,6 +171,7 @@ __device__ __forceinline__ void fft_body(const FftDesc& d, const void* in_, void
       const T s = ((const T*)d.sn)[li.sn + (int64_t)t * d.sn_t_stride];
       v.x *= s; v.y *= s;
     }
+    if (d.mod && d.sign < 0) v = cmul_fma(v, ((const C*)d.mod)[t]);
     out[li.dst + (int64_t)t * d.dst.t_stride] = mk<T>(v.x * scale, v.y * scale_im);
   }
 }

@@ -291,6 +291,14 @@ __device__ __forceinline__ void fft_ct_body(const FftDesc& d, const void* in_, v
       T s[L];
 #pragma unroll
       for (int r = 0; r < L; ++r) v[r] = *(act && j + r * NB0 < d.n_in ? p + r * inc : in);
+      if (d.mod && d.sign > 0) {
+        const C* mod = (const C*)d.mod;
+        C m[L];
+#pragma unroll
+        for (int r = 0; r < L; ++r) m[r] = mod[min(j + r * NB0, N - 1)];
+#pragma unroll
+        for (int r = 0; r < L; ++r) { m[r].y = -m[r].y; v[r] = cmul_fma(v[r], m[r]); }
+      }
       if (d.sn_side == 1) {
         const T* sn = (const T*)d.sn;
         const int64_t s0 = li.sn + (int64_t)(act ? j : 0) * d.sn_t_stride;
@@ -357,6 +365,14 @@ __device__ __forceinline__ void fft_ct_body(const FftDesc& d, const void* in_, v
         s[r] = sn[(int64_t)(o + r * step < d.n_out ? o + r * step : 0) * d.sn_t_stride];
 #pragma unroll
       for (int r = 0; r < R; ++r) { v[r].x *= s[r]; v[r].y *= s[r]; }
+    }
+    if (d.mod && d.sign < 0) {
+      const C* mod = (const C*)d.mod;
+      C m[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) m[r] = mod[o + r * step];
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = cmul_fma(v[r], m[r]);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r)

@@ -25,7 +25,7 @@ int pnh_cast_mul_sn(const void* in, void* out, const float* sn, int64_t n_img, i
 // out[i] = a[i] * b[i]
 int pnh_cmul_c64(const void* a, const void* b, void* out, int64_t n, hipStream_t s);
 // w[i] = |k[i * nb]| (first coil)
-int pnh_abs_first_coil(const void* k, float* w, int64_t n, int nb, hipStream_t s);
+int pnh_abs_first_coil(int fp64, const void* k, float* w, int64_t n, int nb, hipStream_t s);
 // uker (complex64) = mu w - lam * Lap on the grid sh; Lap = lap (complex64)
 // or, with lap null, sum_d 2 cos(2 pi k_d / K_d) - 2
 int pnh_l1tv_uker(const float* w, const void* lap, void* uker, const ShapeArgs& sh, float mu,

@@ -86,11 +86,12 @@ __global__ void cmul_kernel(const float2* __restrict__ a, const float2* __restri
   }
 }
 
-__global__ void abs_kernel(const float2* __restrict__ k, float* __restrict__ w, int64_t n,
-                           int nb) {
+template <typename T>
+__global__ void abs_kernel(const typename cplx<T>::t* __restrict__ k, float* __restrict__ w,
+                           int64_t n, int nb) {
   GRID_STRIDE(i, n) {
-    const float2 v = k[i * nb];
-    w[i] = hypotf(v.x, v.y);
+    const typename cplx<T>::t v = k[i * nb];
+    w[i] = (float)hypot(v.x, v.y);
   }
 }
 
@@ -239,8 +240,9 @@ int pnh_cmul_c64(const void* a, const void* b, void* out, int64_t n, hipStream_t
   return 0;
 }
 
-int pnh_abs_first_coil(const void* k, float* w, int64_t n, int nb, hipStream_t s) {
-  LAUNCH(abs_kernel, n, (const float2*)k, w, n, nb);
+int pnh_abs_first_coil(int fp64, const void* k, float* w, int64_t n, int nb, hipStream_t s) {
+  if (fp64) LAUNCH(abs_kernel<double>, n, (const double2*)k, w, n, nb);
+  else LAUNCH(abs_kernel<float>, n, (const float2*)k, w, n, nb);
   return 0;
 }
 

@@ -41,12 +41,13 @@ int pnh_zero(int fp64, void* p, int64_t n, hipStream_t s);
 int pnh_cg_dot(int mode, const void* a, const void* b, int64_t n_cells, int nb,
                void* part, const int* skip, hipStream_t s);
 // tolerance, first rr and stopping state from the |b|^2 block partials
-int pnh_cg_init(const void* part, int nb, CgScalars* sc, int maxiter, double rtol,
+// part: `blocks` block partials of |b|^2
+int pnh_cg_init(const void* part, int blocks, int nb, CgScalars* sc, int maxiter, double rtol,
                 double atol, hipStream_t s);
 // iteration it: rr from the previous |r|^2 partials rr_part (it > 0), the
 // stopping test, then p = r or p = r + beta p
 int pnh_cg_p_update(void* p, const void* r, int64_t n_cells, int nb, CgScalars* sc,
-                    const void* rr_part, int it, hipStream_t s);
+                    const void* rr_part, int rr_blocks, int it, hipStream_t s);
 // alpha = rr / (p.q) with p.q summed from the block partials pq_part (every
 // workgroup sums them itself); x += alpha p; r -= alpha q; |r|^2 partials
 int pnh_cg_xr_update(void* x, void* r, const void* p, const void* q, int64_t n_cells,
@@ -55,5 +56,5 @@ int pnh_cg_xr_update(void* x, void* r, const void* p, const void* q, int64_t n_c
 // out[c] = ||r|| of coil c at the end of the solve: the value of its
 // stopping test, or (a coil that ran out of iterations) the norm summed from
 // the |r|^2 partials rr_part of the last x/r update (of b when maxiter = 0)
-int pnh_cg_resid(const void* rr_part, int nb, const CgScalars* sc, double* out,
+int pnh_cg_resid(const void* rr_part, int blocks, int nb, const CgScalars* sc, double* out,
                  hipStream_t s);

@@ -3,6 +3,7 @@
 // blocks, each summing a fixed strided subset in a fixed order and reducing
 // in LDS, then one block summing the partials in block order.
 #include "common.h"
+#include "reduce.h"
 #include "vec.h"
 
 namespace {
@@ -100,7 +101,7 @@ dot_partials_kernel(const double2* __restrict__ a, const double2* __restrict__ b
                     int64_t n_cells, int nb, double2* __restrict__ part,
                     const int* __restrict__ skip) {
   if (skip && *skip) return;
-  __shared__ double2 red[256];
+  __shared__ double2 red[4];
   for (int c = 0; c < nb; ++c) {
     double sx = 0.0, sy = 0.0;
     for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < n_cells;
@@ -114,17 +115,8 @@ dot_partials_kernel(const double2* __restrict__ a, const double2* __restrict__ b
         sx += u.x * u.x + u.y * u.y;
       }
     }
-    red[threadIdx.x] = make_double2(sx, sy);
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if ((int)threadIdx.x < s) {
-        red[threadIdx.x].x += red[threadIdx.x + s].x;
-        red[threadIdx.x].y += red[threadIdx.x + s].y;
-      }
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) part[(int64_t)blockIdx.x * nb + c] = red[0];
-    __syncthreads();
+    const double2 tot = sum_block256(make_double2(sx, sy), red);
+    if (threadIdx.x == 0) part[(int64_t)blockIdx.x * nb + c] = tot;
   }
 }
 
@@ -138,17 +130,7 @@ __device__ double2 sum_partials(const double2* __restrict__ part, int nblk, int 
     const double2 v = part[(int64_t)i * nb + c];
     sx += v.x; sy += v.y;
   }
-  red[threadIdx.x] = make_double2(sx, sy);
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st) {
-      red[threadIdx.x].x += red[threadIdx.x + st].x;
-      red[threadIdx.x].y += red[threadIdx.x + st].y;
-    }
-    __syncthreads();
-  }
-  const double2 tot = red[0];
-  __syncthreads();   // red may be reused right away
+  const double2 tot = sum_block256(make_double2(sx, sy), red);
   return tot;
 }
 
@@ -158,7 +140,7 @@ __device__ double2 sum_partials(const double2* __restrict__ part, int nblk, int 
 __global__ void __launch_bounds__(256)
 cg_init_kernel(const double2* __restrict__ part, int nblk, int nb,
                CgScalars* __restrict__ s, int maxiter, double rtol, double atol) {
-  __shared__ double2 red[256];
+  __shared__ double2 red[4];
   const int c = blockIdx.x;
   const double2 tot = sum_partials(part, nblk, nb, c, red);
   if (threadIdx.x != 0) return;
@@ -178,7 +160,7 @@ cg_init_kernel(const double2* __restrict__ part, int nblk, int nb,
 __global__ void __launch_bounds__(256)
 cg_resid_kernel(const double2* __restrict__ part, int nblk, int nb,
                 const CgScalars* __restrict__ s, double* __restrict__ out) {
-  __shared__ double2 red[256];
+  __shared__ double2 red[4];
   const int c = blockIdx.x;
   if (s->stopped[c]) {
     if (threadIdx.x == 0) out[c] = s->res[c];
@@ -205,8 +187,8 @@ __global__ void cg_all_done_kernel(CgScalars* __restrict__ s, int nb) {
 __global__ void __launch_bounds__(256)
 cg_p_update_kernel(double2* __restrict__ p, const double2* __restrict__ r,
                    int64_t n_cells, int nb, CgScalars* __restrict__ s,
-                   const double2* __restrict__ rr_part, int it) {
-  __shared__ double2 red[256];
+                   const double2* __restrict__ rr_part, int rr_blocks, int it) {
+  __shared__ double2 red[4];
   __shared__ double beta[PNH_CG_MAXNB];
   __shared__ int skip[PNH_CG_MAXNB];
   const int ob = (it + 1) & 1, nbuf = it & 1;
@@ -215,13 +197,21 @@ cg_p_update_kernel(double2* __restrict__ p, const double2* __restrict__ r,
     if (writer) s->all_done[nbuf] = 1;
     return;
   }
+  // the first element is under way before the sums
+  const int64_t n = n_cells * nb;
+  const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  double2 r0 = make_double2(0.0, 0.0), p0 = r0;
+  if (first < n) {
+    r0 = r[first];
+    if (it > 0) p0 = p[first];
+  }
   for (int c = 0; c < nb; ++c) {
     const int dold = s->done[ob][c];
     const double rr_old = s->rr[ob][c];
     double rr_new = rr_old;
     int dnew = dold;
     if (it > 0 && !dold) {
-      rr_new = sum_partials(rr_part, PNH_RED_BLOCKS, nb, c, red).x;
+      rr_new = sum_partials(rr_part, rr_blocks, nb, c, red).x;
       dnew = sqrt(rr_new) < s->tol[c];
     }
     if (threadIdx.x == 0) {
@@ -244,15 +234,13 @@ cg_p_update_kernel(double2* __restrict__ p, const double2* __restrict__ r,
     for (int c = 0; c < nb; ++c) all &= skip[c];
     s->all_done[nbuf] = all;
   }
-  const int64_t n = n_cells * nb;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t i = first; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const int c = (int)(i % nb);
     if (skip[c]) continue;
-    const double2 rv = r[i];
+    const double2 rv = i == first ? r0 : r[i];
     if (it == 0) { p[i] = rv; continue; }
     const double bt = beta[c];
-    double2 pv = p[i];
+    double2 pv = i == first ? p0 : p[i];
     pv.x = rv.x + bt * pv.x;
     pv.y = rv.y + bt * pv.y;
     p[i] = pv;
@@ -269,7 +257,7 @@ cg_xr_update_kernel(double2* __restrict__ x, double2* __restrict__ r,
                     const double2* __restrict__ pq_part, int pq_blocks,
                     double2* __restrict__ part) {
   if (s->all_done[buf]) return;
-  __shared__ double2 red[256];
+  __shared__ double2 red[4];
   for (int c = 0; c < nb; ++c) {
     double acc = 0.0;
     if (!s->done[buf][c]) {
@@ -291,14 +279,8 @@ cg_xr_update_kernel(double2* __restrict__ x, double2* __restrict__ r,
         acc += rv.x * rv.x + rv.y * rv.y;
       }
     }
-    red[threadIdx.x] = make_double2(acc, 0.0);
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-      if ((int)threadIdx.x < st) red[threadIdx.x].x += red[threadIdx.x + st].x;
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) part[(int64_t)blockIdx.x * nb + c] = red[0];
-    __syncthreads();
+    const double2 tot = sum_block256(make_double2(acc, 0.0), red);
+    if (threadIdx.x == 0) part[(int64_t)blockIdx.x * nb + c] = tot;
   }
 }
 
@@ -387,10 +369,10 @@ int pnh_cg_dot(int mode, const void* a, const void* b, int64_t n_cells, int nb,
   return 0;
 }
 
-int pnh_cg_init(const void* part, int nb, CgScalars* sc, int maxiter, double rtol,
+int pnh_cg_init(const void* part, int blocks, int nb, CgScalars* sc, int maxiter, double rtol,
                 double atol, hipStream_t s) {
   hipLaunchKernelGGL(cg_init_kernel, dim3(nb), dim3(256), 0, s, (const double2*)part,
-                     PNH_RED_BLOCKS, nb, sc, maxiter, rtol, atol);
+                     blocks, nb, sc, maxiter, rtol, atol);
   PNH_LAUNCH_CHECK();
   if (nb > 1) {
     hipLaunchKernelGGL(cg_all_done_kernel, dim3(1), dim3(64), 0, s, sc, nb);
@@ -400,10 +382,10 @@ int pnh_cg_init(const void* part, int nb, CgScalars* sc, int maxiter, double rto
 }
 
 int pnh_cg_p_update(void* p, const void* r, int64_t n_cells, int nb, CgScalars* sc,
-                    const void* rr_part, int it, hipStream_t s) {
+                    const void* rr_part, int rr_blocks, int it, hipStream_t s) {
   hipLaunchKernelGGL(cg_p_update_kernel, dim3(grid_for(n_cells * nb)), dim3(256), 0, s,
                      (double2*)p, (const double2*)r, n_cells, nb, sc,
-                     (const double2*)rr_part, it);
+                     (const double2*)rr_part, rr_blocks, it);
   PNH_LAUNCH_CHECK();
   return 0;
 }
@@ -419,10 +401,10 @@ int pnh_cg_xr_update(void* x, void* r, const void* p, const void* q, int64_t n_c
   return 0;
 }
 
-int pnh_cg_resid(const void* rr_part, int nb, const CgScalars* sc, double* out,
+int pnh_cg_resid(const void* rr_part, int blocks, int nb, const CgScalars* sc, double* out,
                  hipStream_t s) {
   hipLaunchKernelGGL(cg_resid_kernel, dim3(nb), dim3(256), 0, s, (const double2*)rr_part,
-                     PNH_RED_BLOCKS, nb, sc, out);
+                     blocks, nb, sc, out);
   PNH_LAUNCH_CHECK();
   return 0;
 }
@@ -448,17 +430,9 @@ __device__ __forceinline__ void seg_range(const BatchProblem& pr, int op, int64_
 }
 
 __device__ __forceinline__ void block_sum2(double sx, double sy, double2* out) {
-  __shared__ double2 red[256];
-  red[threadIdx.x] = make_double2(sx, sy);
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st) {
-      red[threadIdx.x].x += red[threadIdx.x + st].x;
-      red[threadIdx.x].y += red[threadIdx.x + st].y;
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = red[0];
+  __shared__ double2 red[4];
+  const double2 tot = sum_block256(make_double2(sx, sy), red);
+  if (threadIdx.x == 0) *out = tot;
 }
 
 // Sum of problem p's block partials (grid table blocks first[p] ..
@@ -472,17 +446,7 @@ __device__ __forceinline__ double2 problem_sum(const double2* __restrict__ part,
     const double2 v = part[i];
     sx += v.x; sy += v.y;
   }
-  red[threadIdx.x] = make_double2(sx, sy);
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st) {
-      red[threadIdx.x].x += red[threadIdx.x + st].x;
-      red[threadIdx.x].y += red[threadIdx.x + st].y;
-    }
-    __syncthreads();
-  }
-  const double2 tot = red[0];
-  __syncthreads();
+  const double2 tot = sum_block256(make_double2(sx, sy), red);
   return tot;
 }
 
@@ -493,7 +457,8 @@ __device__ __forceinline__ double2 problem_sum(const double2* __restrict__ part,
 __global__ void __launch_bounds__(256)
 batch_vec_kernel(int op, const BatchProblem* __restrict__ probs, BatchTable t,
                  int64_t chunk, void* a_, void* b_, void* c_, void* d_, BatchCg cg, int it) {
-  __shared__ double2 red[256];
+  const BatchTable& rt = cg.rr_t;                  // the |r|^2 partials' table
+  __shared__ double2 red[4];
   const int p = t.tab[blockIdx.x];
   const int64_t lb = (int64_t)blockIdx.x - t.first[p];
   const BatchProblem& pr = probs[p];
@@ -505,7 +470,7 @@ batch_vec_kernel(int op, const BatchProblem* __restrict__ probs, BatchTable t,
   if (op == BVEC_P_UPDATE) {
     double beta = 0.0;
     if (it == 0) {
-      const double bb = problem_sum(cg.part_rr, t, p, red).x;
+      const double bb = problem_sum(cg.part_rr, rt, p, red).x;
       const double bn = sqrt(bb);
       const double tol = fmax(cg.atol, cg.rtol * bn);
       const int dn = (bn == 0.0) || (bn < tol);
@@ -527,7 +492,7 @@ batch_vec_kernel(int op, const BatchProblem* __restrict__ probs, BatchTable t,
         }
         return;
       }
-      const double rr_new = problem_sum(cg.part_rr, t, p, red).x;
+      const double rr_new = problem_sum(cg.part_rr, rt, p, red).x;
       const int dn = sqrt(rr_new) < cg.tol[p];
       if (writer) {
         cg.rr[cur * cg.n + p] = rr_new;
@@ -617,14 +582,15 @@ batch_vec_kernel(int op, const BatchProblem* __restrict__ probs, BatchTable t,
 // One block per problem: iterations and final ||r|| (the stopping test's
 // value, else the norm from the last |r|^2 partials; ||b|| at maxiter 0).
 __global__ void __launch_bounds__(256)
-batch_cg_out_kernel(BatchTable t, BatchCg cg, int* __restrict__ iters_out,
+batch_cg_out_kernel(BatchCg cg, int* __restrict__ iters_out,
                     double* __restrict__ resid_out) {
-  __shared__ double2 red[256];
+  __shared__ double2 red[4];
+  const BatchTable& rt = cg.rr_t;
   const int p = blockIdx.x;
   const bool stopped = cg.maxiter > 0 && cg.stopped[p];
   double res = 0.0;
   if (stopped) res = cg.res[p];
-  else res = sqrt(problem_sum(cg.part_rr, t, p, red).x);
+  else res = sqrt(problem_sum(cg.part_rr, rt, p, red).x);
   if (threadIdx.x != 0) return;
   if (iters_out) iters_out[p] = cg.maxiter > 0 ? cg.iters[p] : 0;
   if (resid_out) resid_out[p] = res;
@@ -642,10 +608,10 @@ int pnh_batch_vec_launch(int op, const BatchProblem* probs, const BatchTable& t,
   return 0;
 }
 
-int pnh_batch_cg_out_launch(const BatchTable& t, const BatchCg& cg, int32_t* iters_out,
+int pnh_batch_cg_out_launch(const BatchCg& cg, int32_t* iters_out,
                             double* resid_out, hipStream_t s) {
   if (!iters_out && !resid_out) return 0;
-  hipLaunchKernelGGL(batch_cg_out_kernel, dim3((unsigned)cg.n), dim3(256), 0, s, t, cg,
+  hipLaunchKernelGGL(batch_cg_out_kernel, dim3((unsigned)cg.n), dim3(256), 0, s, cg,
                      iters_out, resid_out);
   PNH_LAUNCH_CHECK();
   return 0;

@@ -312,7 +312,18 @@ def sort_and_bin(base, Kd, Jd, tile, chunk_rows=None):
     counts = np.bincount(tkey, minlength=n_tiles).astype(np.int64)
     starts = np.cumsum(counts) - counts
     if chunk_rows is None:
-        chunk_rows = int(min(MAX_ITEM_ROWS, max(256, math.ceil(M / 2048))))
+        # about 2048 items, but 256 rows at least; 512 where the tiles are many
+        # and full: a box costs its zeroing, its writing and its part of the
+        # gather whatever its rows (512x512, 205 824 samples: adjoint 32 us
+        # with 256 rows, 29 with 512; 120x150x108 grid, 300 007: pair 193,
+        # 168), and a sparse tile's one workgroup takes longer with more
+        # (390x462 grid, 60 001: pair 50 us, 57).  More than 512 would cost
+        # complex64 sums their precision (the fixed point spans the largest
+        # cell that an item's rows can reach)
+        chunk_rows = max(256, math.ceil(M / 2048))
+        if n_tiles >= 512 and M > 160 * n_tiles:
+            chunk_rows = max(chunk_rows, 512)
+        chunk_rows = int(min(MAX_ITEM_ROWS, chunk_rows))
     chunk_rows = int(chunk_rows)
     if not 1 <= chunk_rows <= MAX_ITEM_ROWS:
         raise ValueError('chunk rows must be in 1..%d' % MAX_ITEM_ROWS)
@@ -478,6 +489,94 @@ def plan(om, Nd, Kd, Jd, ft_axes=None, tile=None, chunk_rows=None, cache_dir=Non
               row_bound=row_sum_bound(ud),
               fp64_ops=needs_fp64_operators(st['sn']))
     return st
+
+
+def grid_modulation(N, K):
+    """exp(i pi (N - 1) t / K), t < K, complex128: the phase of a min-max factor
+    as a function of its grid cell (see ``real_records``)."""
+    return np.exp(1j * np.pi * (N - 1) / K * np.arange(K))
+
+
+def _real_chunk(st, rows, check=False):
+    """Real factors c_d (rows, J_d) float64 per axis, and (with ``check``) the
+    largest imaginary part left over relative to the largest factor."""
+    cs, left = [], 0.0
+    for a in range(len(st['Nd'])):
+        N, J, K = st['Nd'][a], st['Jd'][a], st['Kd'][a]
+        u = st['ud'][a][rows]
+        w = np.exp(1j * (st['om'][rows, a] / 2 + np.pi * (N - 1) / K * st['base'][a][rows]))
+        w = w[:, None] * np.exp(1j * np.pi * (N - 1) / K * np.arange(J))[None, :]
+        c = u.real * w.real + u.imag * w.imag
+        if check and u.size:
+            im = np.abs(u.imag * w.real - u.real * w.imag).max()
+            left = max(left, im / max(np.abs(c).max(), 1e-300))
+        cs.append(c)
+    return cs, left
+
+
+# largest imaginary part (relative) of factors taken as real; FP64 rounding
+# leaves 1e-15 to 1e-13
+_REAL_TOL = 1e-10
+
+
+def has_real_factors(st):
+    """Whether the plan's factors are u_j = c_j e^{i om/2} e^{i pi (N-1)(b+j)/K}
+    with c_j real (true of every min-max design: T and r are real), checked on
+    up to 4096 rows."""
+    M = int(st['M'])
+    if M == 0:
+        return True
+    rows = np.unique(np.linspace(0, M - 1, min(M, 4096)).astype(np.int64))
+    return _real_chunk(st, rows, check=True)[1] <= _REAL_TOL
+
+
+def real_records(st, fp64=False, chunk=1 << 15):
+    """Row records of the real factors (include/pynufft_hip.h,
+    ``pnh_real_factors``): (M, W) float32, or (M, V) float64 and the (M,)
+    complex128 phase.  Rows are in gridding order; the chunks run on a thread
+    pool (numpy releases the GIL)."""
+    d, M = len(st['Nd']), int(st['M'])
+    sj = sum(st['Jd'])
+    perm, tile, Kd = st['perm'], st['tile'], st['Kd']
+    if fp64:
+        rec = np.zeros((max(M, 1), (sj + 2) & ~1))
+        phase = np.ones(max(M, 1), np.complex128)
+    else:
+        rec = np.zeros((max(M, 1), (sj + 4 + (d == 3) + 3) & ~3), np.float32)
+    bits = rec.view(np.int64 if fp64 else np.int32)
+
+    def job(s):
+        rows = perm[s:s + chunk]
+        out = rec[s:s + chunk]
+        at = 0
+        for c in _real_chunk(st, rows)[0]:
+            out[:, at:at + c.shape[1]] = c
+            at += c.shape[1]
+        x = [st['base'][a][rows] % tile[a] if tile[a] < Kd[a] else st['base'][a][rows]
+             for a in range(d)]
+        half = st['om'][rows].sum(axis=1) / 2
+        b = bits[s:s + chunk]
+        first = x[0] if d == 1 else x[0] | x[1] << 16
+        if fp64:
+            b[:, at] = first if d < 3 else first | x[2] << 32
+            phase[s:s + chunk] = np.exp(1j * half)
+            return
+        out[:, at] = np.cos(half)
+        out[:, at + 1] = np.sin(half)
+        b[:, at + 2] = first.astype(np.uint32).view(np.int32)
+        if d == 3:
+            b[:, at + 3] = x[2]
+        b[:, at + 3 + (d == 3)] = rows
+
+    starts = range(0, M, chunk)
+    if len(starts) > 1:
+        workers = max(1, min(16, len(os.sched_getaffinity(0))))
+        with concurrent.futures.ThreadPoolExecutor(workers) as pool:
+            list(pool.map(job, starts))
+    else:
+        for s in starts:
+            job(s)
+    return (rec, phase) if fp64 else rec
 
 
 # Apodization spread max|sn| / min|sn| above which the complex64 operators

@@ -161,24 +161,28 @@ class NUFFT:
         # (at least one element each, so that M = 0 still passes valid pointers)
         t['perm'] = torch.from_numpy(
             perm.astype(np.int32) if M else np.zeros(1, np.int32)).to(dev)
-        t['base'] = torch.from_numpy(
-            np.ascontiguousarray(st['base'][:, perm]).astype(np.int32)
-            if M else np.zeros(dd, np.int32)).to(dev)
-        u_sorted = [np.ascontiguousarray(st['ud'][a][perm]) for a in range(dd)]
         self._u_off = [0] * _lib.MAXD
         off = 0
         for a in range(dd):
             self._u_off[a] = off
-            off += u_sorted[a].size
-        u128 = np.concatenate([u.ravel() for u in u_sorted]) if M else \
-            np.zeros(1, np.complex128)
-        t['u_c64'] = torch.from_numpy(u128.astype(np.complex64)).to(dev)
-        self._u128_host = u128
+            off += M * Jd[a]
+        # real factors (one record per row) for the per-axis format; the
+        # complex factors serve the coefficient table and, on demand, the
+        # trajectory's gradient
+        self._real = self._format == 'factor' and helper.has_real_factors(st)
         # apodization spread too large for FP32 operators (Kd close to Nd):
         # forward/adjoint/selfadjoint and the complex64 stages run in FP64
         self.fp64_ops = bool(st.get('fp64_ops', False))
+        if self._real:
+            t['rec_f32'] = torch.from_numpy(helper.real_records(st)).to(dev)
+            for a in range(dd):
+                mod = torch.from_numpy(helper.grid_modulation(Nd[a], Kd[a])).to(dev)
+                t['mod128_%d' % a] = mod
+                t['mod64_%d' % a] = mod.to(_c64)
+        else:
+            self._upload_factors()
         if self.fp64_ops:
-            t['u_c128'] = torch.from_numpy(u128).to(dev)
+            self._upload_fp64()
         t['sn_f32'] = torch.from_numpy(st['sn'].astype(np.float32).ravel()).to(dev)
         t['sn_f64'] = torch.from_numpy(st['sn'].astype(np.float64).ravel()).to(dev)
         for a in range(dd):
@@ -212,6 +216,7 @@ class NUFFT:
         if 'du_c64' not in self._t:
             st = self._host
             perm = st['perm']
+            self._upload_factors()
             du = helper.factor_gradients(st)
             flat = np.concatenate([np.ascontiguousarray(du[a][perm]).ravel()
                                    for a in range(self.ndims)]) if self.M[0] else \
@@ -220,9 +225,47 @@ class NUFFT:
             self._create()
 
     def _ensure_fp64(self):
-        if 'u_c128' not in self._t:
-            self._t['u_c128'] = torch.from_numpy(self._u128_host).to(self.device)
+        if ('rec_f64' if self._real else 'u_c128') not in self._t:
+            self._upload_fp64()
             self._create()
+
+    def _factors128(self):
+        """Per-axis complex128 factors in row order, concatenated."""
+        st = self._host
+        if not self.M[0]:
+            return np.zeros(1, np.complex128)
+        return np.concatenate([st['ud'][a][st['perm']].ravel() for a in range(self.ndims)])
+
+    def _upload_factors(self):
+        """Complex64 factors and first support cells, in row order."""
+        if 'u_c64' in self._t:
+            return
+        st = self._host
+        self._t['u_c64'] = torch.from_numpy(self._factors128().astype(np.complex64)).to(self.device)
+        self._t['base'] = torch.from_numpy(
+            np.ascontiguousarray(st['base'][:, st['perm']]).astype(np.int32)
+            if self.M[0] else np.zeros(self.ndims, np.int32)).to(self.device)
+
+    def _complex_desc(self):
+        """The plan descriptor with complex factors of both precisions (a batch
+        in which some problem has no real factors)."""
+        self._upload_factors()
+        if 'u_c128' not in self._t:
+            self._t['u_c128'] = torch.from_numpy(self._factors128()).to(self.device)
+        d = _lib.PlanDesc.from_buffer_copy(self._desc)
+        d.base = self._t['base'].data_ptr()
+        d.u_c64 = self._t['u_c64'].data_ptr()
+        d.u_c128 = self._t['u_c128'].data_ptr()
+        return d
+
+    def _upload_fp64(self):
+        """What the FP64 operators read: complex128 records or factors."""
+        if self._real:
+            rec, phase = helper.real_records(self._host, fp64=True)
+            self._t['rec_f64'] = torch.from_numpy(rec).to(self.device)
+            self._t['phase_f64'] = torch.from_numpy(phase).to(self.device)
+        else:
+            self._t['u_c128'] = torch.from_numpy(self._factors128()).to(self.device)
 
     def _build_csr(self):
         """Full prod(Jd) coefficient table from the FP64 factors (rounded to
@@ -279,8 +322,8 @@ class NUFFT:
             d.tw_c128[a] = t['tw128_%d' % a].data_ptr()
             d.tile[a] = st['tile'][a]
         d.perm = t['perm'].data_ptr()
-        d.base = t['base'].data_ptr()
-        d.u_c64 = t['u_c64'].data_ptr()
+        d.base = t['base'].data_ptr() if 'base' in t else None
+        d.u_c64 = t['u_c64'].data_ptr() if 'u_c64' in t else None
         d.u_c128 = t['u_c128'].data_ptr() if 'u_c128' in t else None
         d.du_c64 = t['du_c64'].data_ptr() if 'du_c64' in t else None
         d.csr_c64 = t['csr_val'].data_ptr() if 'csr_val' in t else None
@@ -298,10 +341,22 @@ class NUFFT:
         d.threads = self._threads
         d.fp64_ops = 1 if getattr(self, 'fp64_ops', False) else 0
         d.item_bound = t['item_bound'].data_ptr() if 'item_bound' in t else None
+        real = None
+        if self._real:
+            real = _lib.RealFactors()
+            real.rec_f32 = t['rec_f32'].data_ptr()
+            if 'rec_f64' in t:
+                real.rec_f64 = t['rec_f64'].data_ptr()
+                real.phase_f64 = t['phase_f64'].data_ptr()
+            for a in range(self.ndims):
+                real.mod_c64[a] = t['mod64_%d' % a].data_ptr()
+                real.mod_c128[a] = t['mod128_%d' % a].data_ptr()
         h = ctypes.c_void_p()
         with torch.cuda.device(self.device):
-            _lib.check(self._libh.pnh_plan_create(ctypes.byref(d), ctypes.byref(h)))
+            _lib.check(self._libh.pnh_plan_create_real(
+                ctypes.byref(d), None if real is None else ctypes.byref(real), ctypes.byref(h)))
         self._desc = d
+        self._real_desc = real
         self._plan = h
         self._ws = {}
 
