@@ -59,14 +59,14 @@ def algorithmic_bytes(kernel, fmt, M, Jd, Kd, nb=1):
 
 def physical_bytes(fmt, M, Jd, Kd, nb=1):
     """Bytes the format must at least move per launch: the factor format
-    reads sum(Jd) complex64 factors per sample instead of prod(Jd)
-    coefficients, plus d first cells, the row->sample index, the samples
-    and the grid once."""
+    reads one record per sample instead of prod(Jd) coefficients (sum(Jd)
+    real factors, phase, first cells and sample index in 32-bit words, whole
+    16-byte units), plus the samples and the grid once."""
     d = len(Kd)
     K = int(np.prod(Kd))
     P = int(np.prod(Jd))
-    coef = P * 12 if fmt == 'CSR' else int(np.sum(Jd)) * 8 + d * 4
-    return M * (coef + 4 + 8 * nb) + K * 8 * nb
+    row = P * 12 + 4 if fmt == 'CSR' else (int(np.sum(Jd)) + 4 + (d == 3) + 3) // 4 * 16
+    return M * (row + 8 * nb) + K * 8 * nb
 
 
 def lds_atomic_floor_ms(M, Jd, nb=1, per_coef=1):
