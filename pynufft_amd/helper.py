@@ -522,7 +522,7 @@ _REAL_TOL = 1e-10
 def has_real_factors(st):
     """Whether the plan's factors are u_j = c_j e^{i om/2} e^{i pi (N-1)(b+j)/K}
     with c_j real (true of every min-max design: T and r are real), checked on
-    up to 4096 rows."""
+    up to 4096 rows (``real_records`` checks the others)."""
     M = int(st['M'])
     if M == 0:
         return True
@@ -534,7 +534,8 @@ def real_records(st, fp64=False, chunk=1 << 15):
     """Row records of the real factors (include/pynufft_hip.h,
     ``pnh_real_factors``): (M, W) float32, or (M, V) float64 and the (M,)
     complex128 phase.  Rows are in gridding order; the chunks run on a thread
-    pool (numpy releases the GIL)."""
+    pool (numpy releases the GIL).  The float32 records are None if a row's
+    factors turn out not to be of that form."""
     d, M = len(st['Nd']), int(st['M'])
     sj = sum(st['Jd'])
     perm, tile, Kd = st['perm'], st['tile'], st['Kd']
@@ -544,12 +545,15 @@ def real_records(st, fp64=False, chunk=1 << 15):
     else:
         rec = np.zeros((max(M, 1), (sj + 4 + (d == 3) + 3) & ~3), np.float32)
     bits = rec.view(np.int64 if fp64 else np.int32)
+    left = [0.0]
 
     def job(s):
         rows = perm[s:s + chunk]
         out = rec[s:s + chunk]
         at = 0
-        for c in _real_chunk(st, rows)[0]:
+        cs, off = _real_chunk(st, rows, check=not fp64)
+        left.append(off)
+        for c in cs:
             out[:, at:at + c.shape[1]] = c
             at += c.shape[1]
         x = [st['base'][a][rows] % tile[a] if tile[a] < Kd[a] else st['base'][a][rows]
@@ -576,7 +580,9 @@ def real_records(st, fp64=False, chunk=1 << 15):
     else:
         for s in starts:
             job(s)
-    return (rec, phase) if fp64 else rec
+    if fp64:
+        return rec, phase
+    return rec if max(left) <= _REAL_TOL else None
 
 
 # Apodization spread max|sn| / min|sn| above which the complex64 operators

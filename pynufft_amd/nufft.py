@@ -174,7 +174,10 @@ class NUFFT:
         # forward/adjoint/selfadjoint and the complex64 stages run in FP64
         self.fp64_ops = bool(st.get('fp64_ops', False))
         if self._real:
-            t['rec_f32'] = torch.from_numpy(helper.real_records(st)).to(dev)
+            rec = helper.real_records(st)
+            self._real = rec is not None
+        if self._real:
+            t['rec_f32'] = torch.from_numpy(rec).to(dev)
             for a in range(dd):
                 mod = torch.from_numpy(helper.grid_modulation(Nd[a], Kd[a])).to(dev)
                 t['mod128_%d' % a] = mod

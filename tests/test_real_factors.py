@@ -54,3 +54,12 @@ def test_other_factors_are_refused():
     st = helper.plan(np.random.default_rng(0).uniform(-3, 3, (50, 1)), (16,), (32,), (4,))
     st['ud'] = [st['ud'][0] * np.exp(0.1j * np.arange(4))]
     assert not helper.has_real_factors(st)
+
+
+def test_one_other_row_is_found():
+    """A row that the sampled check misses."""
+    st = helper.plan(np.random.default_rng(0).uniform(-3, 3, (9000, 1)), (16,), (32,), (4,))
+    st['ud'][0][8002] *= np.exp(0.1j * np.arange(4))
+    sampled = np.unique(np.linspace(0, 8999, 4096).astype(np.int64))
+    assert 8002 not in sampled and helper.has_real_factors(st)
+    assert helper.real_records(st) is None
